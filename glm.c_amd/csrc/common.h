@@ -53,6 +53,16 @@ __device__ static inline void dma16_untracked(const GM_GLOBAL void *src, lds_voi
     const unsigned m0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)dst);
     asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(m0) : "memory", "m0");
 }
+// The same, BYTES (4 or 16) per lane, from the scalar address base plus the lane's byte offset,
+// so that stepping base along a row costs no vector instruction.
+template <int BYTES>
+__device__ static inline void dma_s(const void *base, unsigned off, const lds_void *dst) {
+    const unsigned m0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)dst);
+    if (BYTES == 16)
+        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
+    else
+        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
+}
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 __host__ __device__ static inline size_t gm_q_offset(int r, int c, int cols) {

@@ -158,13 +158,6 @@ __device__ static inline qg_h4 qg_i8_to_h4(unsigned u) {
     return r;
 }
 
-// 4 bytes from global memory into shared memory: lane l's at dst + 4 l, by a DMA that the
-// compiler does not count (the caller waits on vmcnt).
-__device__ static inline void dma4_untracked(const GM_GLOBAL void *src, lds_void *dst) {
-    const unsigned m0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)dst);
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(m0) : "memory", "m0");
-}
-
 // One stage of the chunk pipeline in shared memory: every operand of a chunk of QG_KC
 // columns arrives by DMA that the compiler does not track, so its only waits are the
 // pipeline's exact vmcnt counts. (Weights loaded into registers instead make the compiler
@@ -182,56 +175,76 @@ struct QgStageBuf {
 };
 
 // Per-thread sources of a tile's DMA: NA activation slots (16 bytes), and for each matrix
-// one weight slot (16 bytes of row t / 4 of the panel) and one scale slot (4 bytes).
+// one weight slot (16 bytes of row t / 4 of the panel) and one scale slot (4 bytes), as
+// offsets of chunk 0 from the tile's first token's split row, the panel's first weight and its
+// first scale; chunk kc's lie QG_KC columns (halves, weights) and QG_KC / KB scales times kc on.
 template <int NA>
 struct QgSrc {
-    const __half *act[NA];  // the slot's activation row at column 0
-    int act_col[NA];        // the slot's first column within a chunk
-    int w_row, w_col;       // panel row (clamped) and column of the weight slot within a chunk
-    int s_row, s_blk;       // panel row (clamped) and block of the scale slot
+    const __half *act0;             // the tile's first token, at the group's first column
+    const int8_t *w0;               // first weight of the panel's first row (of the first matrix)
+    const float *s0;                // first scale of the panel's first row
+    ptrdiff_t dw, ds;               // the second matrix's distance
+    unsigned act[NA], wo, so;       // the slots' byte offsets
+    unsigned short col[NA];         // the activation slots' first columns within a chunk
+    unsigned short w_col, s_blk;    // the weight slot's first column and the scale slot's group
 };
 
-template <int NA, int KB>
+template <int NA, int KB, int NM>
 __device__ static inline QgSrc<NA> qg_src_init(const QgArgs &a, int t0, int c_off, int row0, int nrows) {
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int tid = threadIdx.x;
+    const int ng = a.cols / KB;
     QgSrc<NA> g;
+    g.act0 = a.xs + (size_t)t0 * 2 * a.xcols + c_off;
+    g.w0 = a.q + (size_t)row0 * a.cols;
+    g.s0 = a.s + (size_t)row0 * ng;
+    g.dw = NM == 2 ? a.q2 - a.q : 0;
+    g.ds = NM == 2 ? a.s2 - a.s : 0;
 #pragma unroll
     for (int it = 0; it < NA; it++) {
-        const int s = 64 * w + QG_BLOCK * it + lane, r = s / QG_RG, p = s % QG_RG, tok = r >> 1;
+        const int s = QG_BLOCK * it + tid, r = s / QG_RG, p = s % QG_RG, tok = r >> 1;
         const int j = p ^ (tok & 7);  // the slot holds logical group j of its row
-        const int t = t0 + tok < a.n ? t0 + tok : a.n - 1;
-        g.act[it] = a.xs + ((size_t)t * 2 + (r & 1)) * a.xcols + c_off;
-        g.act_col[it] = 8 * j;
+        const int t = t0 + tok < a.n ? tok : a.n - 1 - t0;
+        g.col[it] = 8 * j;
+        g.act[it] = 2u * ((2u * t + (r & 1)) * a.xcols + 8 * j);
     }
     const int wr = tid >> 2, wg = (tid & 3) ^ ((wr >> 2) & 3);  // slot tid holds group wg of row wr
-    g.w_row = row0 + (wr < nrows ? wr : 0);
     g.w_col = 16 * wg;
+    g.wo = (unsigned)(wr < nrows ? wr : 0) * a.cols + 16 * wg;
     constexpr int NB = QG_KC / KB;
-    const int sr = tid / NB;
-    g.s_row = row0 + (sr < nrows ? sr : 0);  // slots past the panel's 64 rows (NB = 2) load row 0
+    const int sr = tid / NB;  // slots past the panel's 64 rows (NB = 2) load row 0
     g.s_blk = tid % NB;
+    g.so = 4u * ((unsigned)(sr < nrows ? sr : 0) * ng + tid % NB);
     return g;
 }
 
 template <int NA, int KB, int NM>
 __device__ static inline void qg_issue(const QgArgs &a, const QgSrc<NA> &g, QgStageBuf<NM> &sb, int c0) {
-    const int w = threadIdx.x >> 6;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const __half *act = g.act0 + c0;
+    const int8_t *wq = g.w0 + c0;
+    const float *ws = g.s0 + c0 / KB;
+    if (c0 + QG_KC <= a.cols) {
+#pragma unroll
+        for (int it = 0; it < NA; it++) dma_s<16>(act, g.act[it], (const lds_void *)(sb.act + 16 * (64 * w + QG_BLOCK * it)));
+#pragma unroll
+        for (int m = 0; m < NM; m++) {
+            dma_s<16>(wq + (m ? g.dw : 0), g.wo, (const lds_void *)(sb.w[m] + 1024 * w));
+            dma_s<4>(ws + (m ? g.ds : 0), g.so, (const lds_void *)(sb.s[m] + 64 * w));
+        }
+        return;
+    }
+    // the last chunk's part past the last column: zeros for the inputs, any weights and scales
 #pragma unroll
     for (int it = 0; it < NA; it++) {
-        const int c = c0 + g.act_col[it];
-        const __half *src = c < a.cols ? g.act[it] + c : a.zeros;  // past the last column: zeros
+        const __half *src = c0 + g.col[it] < a.cols ? (const __half *)((const char *)act + g.act[it]) : a.zeros;
         dma16_untracked(gbl((const void *)src), (lds_void *)(sb.act + 16 * (64 * w + QG_BLOCK * it)));
     }
-    const int ng = a.cols / a.gs;
-    const int cw = c0 + g.w_col < a.cols ? c0 + g.w_col : 0;  // past the last column: any weights
-    const int cs = c0 + KB * g.s_blk;
-    const int gi = cs < a.cols ? cs / a.gs : 0;
+    const unsigned wo = c0 + g.w_col < a.cols ? g.wo : g.wo - g.w_col;
+    const unsigned so = c0 + KB * g.s_blk < a.cols ? g.so : g.so - 4 * g.s_blk;
 #pragma unroll
     for (int m = 0; m < NM; m++) {
-        const int8_t *q = m ? a.q2 : a.q;
-        const float *s = m ? a.s2 : a.s;
-        dma16_untracked(gbl((const void *)(q + (size_t)g.w_row * a.cols + cw)), (lds_void *)(sb.w[m] + 1024 * w));
-        dma4_untracked(gbl((const void *)(s + (size_t)g.s_row * ng + gi)), (lds_void *)(sb.s[m] + 64 * w));
+        dma_s<16>(wq + (m ? g.dw : 0), wo, (const lds_void *)(sb.w[m] + 1024 * w));
+        dma_s<4>(ws + (m ? g.ds : 0), so, (const lds_void *)(sb.s[m] + 64 * w));
     }
 }
 
@@ -254,43 +267,62 @@ __device__ static inline const uint8_t *qg_w(const uint8_t *w, int r, int c) {
     return w + r * QG_KC + 16 * g + (c & 15);
 }
 
+// The chunk's products: every operand is read from shared memory before the first is used (a
+// read's latency is paid once a chunk, not once a block), and the MFMAs of different blocks
+// and A tiles, which do not depend on each other, lie between a hi product and its lo.
 template <int NA, int KB>
-__device__ static inline void qg_mma(const uint8_t *act, const uint8_t *wm, const float *sm, const QgArgs &a, int c0,
-                                     int r, float (*acc)[4]) {
+__device__ static inline void qg_mma(const uint8_t *act, const uint8_t *wm, const float *sm, int left, int r, float (*acc)[4]) {
     const qg_f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
     const int lane = threadIdx.x & 63;
     constexpr int NB = QG_KC / KB;
+    typedef typename std::conditional<KB == 32, qg_h8, qg_h4>::type frag;
+    typedef typename std::conditional<KB == 32, qg_u2, unsigned>::type raw;
+    raw q[NB];
+    float sc[NB];
+    frag A[2][NB][NA];
+#pragma unroll
+    for (int b = 0; b < NB; b++) q[b] = *(const raw *)qg_w(wm, r, KB * b + KB / 4 * (lane >> 4));
+#pragma unroll
+    for (int b = 0; b < NB; b++) sc[b] = sm[r * NB + b];
+#pragma unroll
+    for (int pl = 0; pl < 2; pl++)
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int i = 0; i < NA; i++) {
+                if constexpr (KB == 32) A[pl][b][i] = qg_a8(act, i, pl, b);
+                else A[pl][b][i] = qg_a4(act, i, pl, b);
+            }
+    frag B[NB];
 #pragma unroll
     for (int b = 0; b < NB; b++) {
-        const float sc = c0 + KB * b < a.cols ? sm[r * NB + b] : 0.0f;
-        if (KB == 32) {
-            const qg_u2 q = *(const qg_u2 *)qg_w(wm, r, 32 * b + 8 * (lane >> 4));
-            const qg_h8 B = qg_i8_to_h8(q.x, q.y);
-#pragma unroll
-            for (int i = 0; i < NA; i++) {
-                qg_f4 d = __builtin_amdgcn_mfma_f32_16x16x32_f16(qg_a8(act, i, 0, b), B, zero, 0, 0, 0);
-                d = __builtin_amdgcn_mfma_f32_16x16x32_f16(qg_a8(act, i, 1, b), B, d, 0, 0, 0);
-#pragma unroll
-                for (int k = 0; k < 4; k++) acc[i][k] = fmaf(d[k], sc, acc[i][k]);
-            }
-        } else {
-            const unsigned q = *(const unsigned *)qg_w(wm, r, 16 * b + 4 * (lane >> 4));
-            const qg_h4 B = qg_i8_to_h4(q);
-#pragma unroll
-            for (int i = 0; i < NA; i++) {
-                qg_f4 d = __builtin_amdgcn_mfma_f32_16x16x16f16(qg_a4(act, i, 0, b), B, zero, 0, 0, 0);
-                d = __builtin_amdgcn_mfma_f32_16x16x16f16(qg_a4(act, i, 1, b), B, d, 0, 0, 0);
-#pragma unroll
-                for (int k = 0; k < 4; k++) acc[i][k] = fmaf(d[k], sc, acc[i][k]);
-            }
-        }
+        if constexpr (KB == 32) B[b] = qg_i8_to_h8(q[b].x, q[b].y);
+        else B[b] = qg_i8_to_h4(q[b]);
+        if (KB * b >= left) sc[b] = 0.0f;  // past the last column
     }
+    qg_f4 d[NB][NA];
+#pragma unroll
+    for (int pl = 0; pl < 2; pl++)
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int i = 0; i < NA; i++) {
+                if constexpr (KB == 32) d[b][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[pl][b][i], B[b], pl ? d[b][i] : zero, 0, 0, 0);
+                else d[b][i] = __builtin_amdgcn_mfma_f32_16x16x16f16(A[pl][b][i], B[b], pl ? d[b][i] : zero, 0, 0, 0);
+            }
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int i = 0; i < NA; i++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) acc[i][k] = fmaf(d[b][i][k], sc[b], acc[i][k]);
 }
 
 // The tile of block (panel, token tile): wave w takes rows 16 w .. +16 of the panel. The
-// chunks run double-buffered: chunk kc + 1's operands are requested before chunk kc is
-// multiplied; each step waits for exactly the loads issued before the prefetch (vmcnt)
-// and then on the block (s_barrier), so the prefetch stays in flight.
+// chunks run double-buffered with one barrier each: a step waits for its own chunk's loads
+// and for the wave's shared-memory reads of the chunk before, then on the block, after which
+// that chunk's stage takes the next chunk while this one is multiplied. (Three, four and six
+// stages measured no faster at 201 and 1024 tokens: what a chunk cost was its instructions.)
 template <int NA, int KB, int MODE, int NM>
 __device__ __attribute__((always_inline)) static void qg_tile(const QgArgs &a, int panel, int tt,
                                                              QgStageBuf<NM> (&buf)[2]) {
@@ -302,8 +334,7 @@ __device__ __attribute__((always_inline)) static void qg_tile(const QgArgs &a, i
     const int pr = 16 * w + (lane & 15);                             // the lane's panel row
     const bool row_on = pr < nrows;
     const int t0 = QG_TT * tt;
-    const QgSrc<NA> src = qg_src_init<NA, KB>(a, t0, g * a.x_stride, row0, nrows);
-    constexpr int LOADS = NA + 2 * NM;  // DMA per chunk and thread
+    const QgSrc<NA> src = qg_src_init<NA, KB, NM>(a, t0, g * a.x_stride, row0, nrows);
     float acc[NA][4], acc2[NA][4];
 #pragma unroll
     for (int i = 0; i < NA; i++)
@@ -311,20 +342,15 @@ __device__ __attribute__((always_inline)) static void qg_tile(const QgArgs &a, i
         for (int k = 0; k < 4; k++) acc[i][k] = acc2[i][k] = 0.0f;
     const int nkc = (a.cols + QG_KC - 1) / QG_KC;
     auto compute = [&](const QgStageBuf<NM> &sb, int kc) {
-        qg_mma<NA, KB>(sb.act, sb.w[0], sb.s[0], a, kc * QG_KC, pr, acc);
-        if (NM == 2) qg_mma<NA, KB>(sb.act, sb.w[NM - 1], sb.s[NM - 1], a, kc * QG_KC, pr, acc2);
+        qg_mma<NA, KB>(sb.act, sb.w[0], sb.s[0], a.cols - kc * QG_KC, pr, acc);
+        if (NM == 2) qg_mma<NA, KB>(sb.act, sb.w[NM - 1], sb.s[NM - 1], a.cols - kc * QG_KC, pr, acc2);
     };
     qg_issue<NA, KB, NM>(a, src, buf[0], 0);
     for (int kc = 0; kc < nkc; kc++) {
-        if (kc + 1 < nkc) {
-            qg_issue<NA, KB, NM>(a, src, buf[(kc + 1) & 1], (kc + 1) * QG_KC);
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
-        } else {
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        }
-        __builtin_amdgcn_s_barrier();  // every wave's part of chunk kc has landed
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();  // chunk kc has landed, and chunk kc - 1 is done with
+        if (kc + 1 < nkc) qg_issue<NA, KB, NM>(a, src, buf[(kc + 1) & 1], (kc + 1) * QG_KC);
         compute(buf[kc & 1], kc);
-        __builtin_amdgcn_s_barrier();  // every wave is done with the stage before its refill
     }
     // lane l holds tokens 16 i + 4 (l / 16) + k of panel row pr
     const int r = row0 + pr;
@@ -368,8 +394,15 @@ __device__ __attribute__((always_inline)) static inline void qg_with_na(int na, 
 // resident together share their tokens' inputs in L2 (walking one panel's tiles before the
 // next streamed the whole input once per panel: 603 MB fetched per attn_out call of a
 // 1024-token batch, for 31.5 MB of weights and inputs).
+// What bounds it is instruction issue: a chunk's eight or sixteen MFMAs take 128 or 256 clocks of a
+// wave, and everything else in it has to stay near that. Hence scalar base addresses stepped
+// along the rows (no vector instruction a DMA, no division by the group size), operands read
+// together, the accumulators in vector registers (launch bounds that leave the matrix cores no
+// use for their own, whose every read is an instruction). Before and after, us: group size 16,
+// 201 tokens: attn_out 74 -> 52, layer 0's gate/up 137 -> 84, q_a 30 -> 22; group size 32, 1024
+// tokens: attn_out 107 -> 98, gate/up 318 -> 275.
 template <int KB, int MODE>
-__global__ __launch_bounds__(QG_BLOCK) void k_gemm_q8(QgArgs a) {
+__global__ __launch_bounds__(QG_BLOCK, MODE == QG_PAIR ? 3 : 4) void k_gemm_q8(QgArgs a) {
     constexpr int NM = MODE == QG_PAIR ? 2 : 1;
     __shared__ __align__(16) QgStageBuf<NM> buf[2];
     const int b = blockIdx.x, xcd = b % QG_XCD, k = b / QG_XCD;

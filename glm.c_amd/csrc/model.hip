@@ -509,8 +509,7 @@ void gemm_launch(gmoe_model *m, const int8_t *q, const float *s, const int8_t *q
     a.tiles = (n + QG_TT - 1) / QG_TT;
     const int panels = a.bpg * a.groups;
     const dim3 grid((unsigned)(QG_XCD * ((panels + QG_XCD - 1) / QG_XCD) * a.tiles));
-    const bool k32 = a.gs % 32 == 0 && cols % 32 == 0;
-    if (k32) {
+    if (a.gs == 32) {  // gemm_batch: 16 or 32, the kernel's block of columns with one scale
         if (mode == QG_PAIR) hipLaunchKernelGGL((k_gemm_q8<32, QG_PAIR>), grid, dim3(QG_BLOCK), 0, st, a);
         else if (mode == QG_RESID) hipLaunchKernelGGL((k_gemm_q8<32, QG_RESID>), grid, dim3(QG_BLOCK), 0, st, a);
         else hipLaunchKernelGGL((k_gemm_q8<32, QG_PLAIN>), grid, dim3(QG_BLOCK), 0, st, a);
