@@ -63,6 +63,24 @@ __device__ static inline void dma_s(const void *base, unsigned off, const lds_vo
     else
         asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
 }
+// N (at most 4) consecutive pieces of 1 KB, 16 bytes per lane each: piece i from base + 1024 i
+// to dst + 1024 i, by the instruction's offset, which applies to both.
+template <int N>
+__device__ static inline void dma_run(const void *base, unsigned off, const lds_void *dst) {
+    const unsigned m0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)dst);
+#define GM_DMA "global_load_lds_dwordx4 %0, %1"
+    if (N == 1)
+        asm volatile("s_mov_b32 m0, %2\n\t" GM_DMA ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
+    else if (N == 2)
+        asm volatile("s_mov_b32 m0, %2\n\t" GM_DMA "\n\t" GM_DMA " offset:1024" ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
+    else if (N == 3)
+        asm volatile("s_mov_b32 m0, %2\n\t" GM_DMA "\n\t" GM_DMA " offset:1024\n\t" GM_DMA " offset:2048" ::"v"(off), "s"(base),
+                     "s"(m0) : "memory", "m0");
+    else
+        asm volatile("s_mov_b32 m0, %2\n\t" GM_DMA "\n\t" GM_DMA " offset:1024\n\t" GM_DMA " offset:2048\n\t" GM_DMA
+                     " offset:3072" ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
+#undef GM_DMA
+}
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 __host__ __device__ static inline size_t gm_q_offset(int r, int c, int cols) {

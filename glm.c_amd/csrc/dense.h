@@ -241,23 +241,21 @@ struct AttnArgs {
     int nblk;              // position ranges of k_attn_chunk (blocks per head group), <= AT_MAX_PARTS
     float kq_scale;
     // this layer's cache entries in split fp16 form for the batch attention on matrix cores
-    // (null: not kept): ksp [cap16][SPL_KROW] halves, a row per position (see below); vsp
-    // [cap16 / 16][2][kv][16] halves, the compressed part transposed in blocks of 16 positions
-    _Float16 *ksp, *vsp;
+    // (null: not kept): [cap32][SPL_KROW] halves, a row per position (see below)
+    _Float16 *ksp;
 };
 
 // The split form of a cache entry (the matrix cores' operands, written once per position
 // by attn_prep_run): x = hi + lo, fp16 each, of the entry scaled by 2^-e, e the exponent with
 // max |entry| 2^-e < 2^15 (SPL_EMPTY for a zero entry). A ksp row is the kv + rope columns'
-// hi (SPL_KCOLS halves, zeros past kv + rope), then their lo, then e (an int), then
-// padding to SPL_KROW halves, an odd count of 16-byte units so that rows read together fall
-// in distinct banks. vsp holds the compressed part's hi and lo planes transposed by blocks
-// of 16 positions: block b, plane, column c, position slot s at ((b * 2 + plane) * kv + c) * 16 + s.
+// hi (SPL_KCOLS halves, zeros past kv + rope), then their lo, then e (an int), then padding
+// to SPL_KROW halves: rows 8 banks apart (of 64), so that the eight rows x 32 bytes that half
+// a wave's transposing load reads (attn16.h) fall in distinct banks, as do eight rows' 16 bytes.
 #define SPL_KCOLS 576
 #define SPL_KEXP (2 * SPL_KCOLS)   // half index of the exponent in a ksp row
-#define SPL_KROW (2 * SPL_KCOLS + 8)
+#define SPL_KROW (2 * SPL_KCOLS + 16)
 #define SPL_EMPTY (-1000)
-static_assert((SPL_KROW * 2 / 16) % 2 == 1, "a ksp row is an odd count of 16-byte units");
+static_assert(SPL_KROW * 2 % 256 == 32 && SPL_KROW * 2 % 16 == 0, "ksp rows lie 8 banks apart");
 
 // The exponent e with |x| 2^-e < 2^15 for every |x| <= mx (SPL_EMPTY when mx is 0).
 __device__ static inline int spl_exp(float mx) {
@@ -274,10 +272,9 @@ __device__ static inline void spl_split(float x, _Float16 &hi, _Float16 &lo) {
 }
 
 // The split form of the entry row[0 .. kv + rope) (the block's shared memory, written before
-// a barrier) into ksp row kr and vsp slot vb (kv + rope <= SPL_KCOLS, kv <= the vsp planes'
-// width: the host's checks); rmax: DM_BLOCK / 64 floats of shared memory.
-__device__ __attribute__((always_inline)) static void spl_store(const float *row, int kv, int rope, _Float16 *kr,
-                                                                _Float16 *vb, float *rmax) {
+// a barrier) into ksp row kr (kv + rope <= SPL_KCOLS: the host's check); rmax: DM_BLOCK / 64
+// floats of shared memory.
+__device__ __attribute__((always_inline)) static void spl_store(const float *row, int kv, int rope, _Float16 *kr, float *rmax) {
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, KQ = kv + rope;
     float mx = 0.0f;
     for (int i = tid; i < KQ; i += DM_BLOCK) mx = fmaxf(mx, fabsf(row[i]));
@@ -290,10 +287,6 @@ __device__ __attribute__((always_inline)) static void spl_store(const float *row
         if (i < KQ) spl_split(ldexpf(row[i], -e), hi, lo);
         kr[i] = hi;
         kr[SPL_KCOLS + i] = lo;
-        if (i < kv) {
-            vb[(size_t)i * 16] = hi;
-            vb[((size_t)kv + i) * 16] = lo;
-        }
     }
     if (tid < (SPL_KROW - SPL_KEXP) / 2) ((int *)(kr + SPL_KEXP))[tid] = tid == 0 ? e : 0;
 }
@@ -346,13 +339,12 @@ __device__ __attribute__((always_inline)) static void attn_prep_run(AttnArgs a, 
     }
     if (!a.ksp) return;  // a decode step: the host marks the position for k_spl_fill
     __syncthreads();
-    spl_store(row, a.kv, a.rope, a.ksp + (size_t)a.pos * SPL_KROW, a.vsp + (size_t)(a.pos >> 4) * 2 * a.kv * 16 + (a.pos & 15),
-              rmax);
+    spl_store(row, a.kv, a.rope, a.ksp + (size_t)a.pos * SPL_KROW, rmax);
 }
 
 // Positions p0 + blockIdx.x of attention layer blockIdx.y: the split form from the fp32
 // entry (the same values attn_prep_run splits), for positions a decode step wrote without it.
-__global__ __launch_bounds__(DM_BLOCK) void k_spl_fill(const float *comp, const float *pe, _Float16 *ksp, _Float16 *vsp,
+__global__ __launch_bounds__(DM_BLOCK) void k_spl_fill(const float *comp, const float *pe, _Float16 *ksp,
                                                       size_t cap, size_t capt, int kv, int rope, int p0) {
     __shared__ float row[SPL_KCOLS];
     __shared__ float rmax[DM_BLOCK / 64];
@@ -360,8 +352,7 @@ __global__ __launch_bounds__(DM_BLOCK) void k_spl_fill(const float *comp, const 
     const float *ce = comp + ((size_t)l * cap + p) * kv, *re = pe + ((size_t)l * cap + p) * rope;
     for (int i = threadIdx.x; i < kv + rope; i += DM_BLOCK) row[i] = i < kv ? ce[i] : re[i - kv];
     __syncthreads();
-    spl_store(row, kv, rope, ksp + ((size_t)l * capt + p) * SPL_KROW,
-              vsp + (size_t)l * capt * 2 * kv + (size_t)(p >> 4) * 2 * kv * 16 + (p & 15), rmax);
+    spl_store(row, kv, rope, ksp + ((size_t)l * capt + p) * SPL_KROW, rmax);
 }
 
 // The query side of a token's attention in one launch: the absorbed queries q_abs = k_b_h .

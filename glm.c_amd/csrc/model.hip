@@ -94,10 +94,10 @@ struct gmoe_model {
     float *x = nullptr, *q_a = nullptr, *q_full = nullptr, *kv_a = nullptr, *q_pe = nullptr, *q_abs = nullptr,
           *ctx = nullptr, *concat = nullptr, *ffh = nullptr, *logits = nullptr, *part_ctx = nullptr,
           *part_ml = nullptr, *saved = nullptr;
-    // the caches' split fp16 form for the batch attention (dense.h: ksp rows, vsp blocks; null
-    // where the shape does not take it), cap rounded up to 16 positions
-    _Float16 *ksp = nullptr, *vsp = nullptr;
-    size_t cap16 = 0;
+    // the caches' split fp16 form for the batch attention (dense.h: ksp rows; null
+    // where the shape does not take it), cap rounded up to whole tiles of A16_P positions
+    _Float16 *ksp = nullptr;
+    size_t cap32 = 0;
     // positions stale_lo .. stale_hi - 1 hold fp32 entries a decode step wrote without their
     // split form (decode reads only the fp32 cache); a prefill converts them first
     int stale_lo = 0, stale_hi = 0;
@@ -320,8 +320,7 @@ AttnArgs attn_args(gmoe_model *m, int l, int pos) {
     aa.part_ctx = m->part_ctx;
     aa.part_ml = m->part_ml;
     aa.ctx = m->ctx;
-    aa.ksp = m->ksp ? m->ksp + (size_t)l * m->cap16 * SPL_KROW : nullptr;
-    aa.vsp = m->vsp ? m->vsp + (size_t)l * m->cap16 * 2 * kv : nullptr;
+    aa.ksp = m->ksp ? m->ksp + (size_t)l * m->cap32 * SPL_KROW : nullptr;
     aa.H = H;
     aa.kv = kv;
     aa.rope = rope;
@@ -393,7 +392,7 @@ void launch_attn_tile(gmoe_model *m, AttnArgs aa, int n, hipStream_t st) {
     const int per = (P + nch - 1) / nch;
     AttnTileArgs g;
     g.n = n;
-    g.chunk = std::max(AQ_P, (per + AQ_P - 1) / AQ_P * AQ_P);
+    g.chunk = std::max(A16_P, (per + A16_P - 1) / A16_P * A16_P);
     aa.nblk = (P + g.chunk - 1) / g.chunk;
     g.a = aa;
     const dim3 grid((unsigned)aa.nblk, (unsigned)tiles, (unsigned)aa.H);
@@ -402,7 +401,7 @@ void launch_attn_tile(gmoe_model *m, AttnArgs aa, int n, hipStream_t st) {
     // reference for the split form)
     const char *env = getenv("GMOE_ATTN_TILE_FP32");
     if (!(env && env[0] == '1') && aa.ksp) {
-        hipLaunchKernelGGL(k_attn_tile16, grid, dim3(AQ_BLOCK), 0, st, g);
+        hipLaunchKernelGGL(k_attn_tile16, grid, dim3(A16_BLOCK), 0, st, g);
     } else {
         switch (aq_rounds(aa.kv + aa.rope)) {
         case 1: hipLaunchKernelGGL(k_attn_tile<1>, grid, dim3(AQ_BLOCK), 0, st, g); break;
@@ -426,7 +425,7 @@ int attention(gmoe_model *m, int l, int pos, hipStream_t st) {
     }
     launch_gemv(gemv(A.q_b_q, A.q_b_s, m->q_a, A.q_a_norm, m->q_full, H * c.head_k_dim, c.q_lora_rank, gs), GV_PLAIN, st);
     AttnArgs aa = attn_args(m, l, pos);
-    aa.ksp = aa.vsp = nullptr;  // the split form waits for the next prefill (k_spl_fill)
+    aa.ksp = nullptr;  // the split form waits for the next prefill (k_spl_fill)
     // the query absorbed into the latent space, per head: k_b_h [kv][nope] . q_nope_h, with
     // the cache entry and the rotated queries in the same launch
     GemvArgs kb = gemv(A.k_b_q, A.k_b_s, m->q_full, nullptr, m->q_abs, H * kv, c.qk_nope_dim, gs);
@@ -653,9 +652,8 @@ extern "C" int gmoe_model_create(gmoe_model **out, int device, const gmoe_model_
         rc |= mdalloc(m, &m->part_ml, ranges * H * 2);
         rc |= mdalloc(m, &m->saved, A * (kv + rope));
         if (attn_tile_ok(c) && kv <= AT_KV_MAX) {
-            m->cap16 = (cap + 15) / 16 * 16;
-            rc |= mdalloc(m, &m->ksp, A * m->cap16 * SPL_KROW);
-            rc |= mdalloc(m, &m->vsp, A * m->cap16 * 2 * kv);
+            m->cap32 = (cap + A16_P - 1) / A16_P * A16_P;
+            rc |= mdalloc(m, &m->ksp, A * m->cap32 * SPL_KROW);
         }
     }
     if (!rc && A > 0) {
@@ -674,8 +672,7 @@ extern "C" int gmoe_model_create(gmoe_model **out, int device, const gmoe_model_
         }
         if (!rc && (hipMemset(m->comp, 0, A * cap * kv * sizeof(float)) != hipSuccess ||
                     hipMemset(m->pe, 0, A * cap * rope * sizeof(float)) != hipSuccess ||
-                    (m->ksp && hipMemset(m->ksp, 0, A * m->cap16 * SPL_KROW * sizeof(_Float16)) != hipSuccess) ||
-                    (m->vsp && hipMemset(m->vsp, 0, A * m->cap16 * 2 * kv * sizeof(_Float16)) != hipSuccess))) {
+                    (m->ksp && hipMemset(m->ksp, 0, A * m->cap32 * SPL_KROW * sizeof(_Float16)) != hipSuccess))) {
             gm_set_err("gmoe_model_create: clearing the cache failed");
             rc = GMOE_ERR_HIP;
         }
@@ -930,7 +927,7 @@ extern "C" int gmoe_model_prefill(gmoe_model *m, const int32_t *tokens, int n, i
         // the entries decode steps wrote without their split form, before any attention of
         // this batch reads them
         hipLaunchKernelGGL(k_spl_fill, dim3((unsigned)(m->stale_hi - m->stale_lo), (unsigned)c.attn_layers), dim3(DM_BLOCK),
-                           0, st, m->comp, m->pe, m->ksp, m->vsp, (size_t)c.cache_cap, m->cap16, c.kv_lora_rank, c.rope_dim,
+                           0, st, m->comp, m->pe, m->ksp, (size_t)c.cache_cap, m->cap32, c.kv_lora_rank, c.rope_dim,
                            m->stale_lo);
         m->stale_lo = m->stale_hi = 0;
     }
