@@ -322,3 +322,36 @@ __device__ static inline float digits_to_float(int D0, int D1, int D2) {
     int lo = D0 + (D1 << 8);  // |lo| < 2^29
     return fmaf((float)D2, 65536.0f, (float)lo);
 }
+
+// ---------------------------------------------------------------- split activations
+//
+// Columns i .. i + 7 of a row of fp32 values in the GEMMs' split form: hi = fp16(v 2^-e) and
+// lo = fp16(v 2^-e - hi), one 16-byte store each.
+__device__ static inline void split8(const float *src, int e, __half *hi, __half *lo) {
+    const float4 a = *(const float4 *)src, b = *(const float4 *)(src + 4);
+    const float xs[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    unsigned hw[4], lw[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const float x0 = ldexpf(xs[2 * k], -e), x1 = ldexpf(xs[2 * k + 1], -e);
+        const __half h0 = __float2half_rn(x0), h1 = __float2half_rn(x1);
+        const __half l0 = __float2half_rn(x0 - __half2float(h0)), l1 = __float2half_rn(x1 - __half2float(h1));
+        hw[k] = (unsigned)__half_as_ushort(h0) | ((unsigned)__half_as_ushort(h1) << 16);
+        lw[k] = (unsigned)__half_as_ushort(l0) | ((unsigned)__half_as_ushort(l1) << 16);
+    }
+    *(uint4 *)hi = make_uint4(hw[0], hw[1], hw[2], hw[3]);
+    *(uint4 *)lo = make_uint4(lw[0], lw[1], lw[2], lw[3]);
+}
+// The largest magnitude of the eight.
+__device__ static inline float absmax8(const float *src) {
+    const float4 a = *(const float4 *)src, b = *(const float4 *)(src + 4);
+    return fmaxf(fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fmaxf(fabsf(a.z), fabsf(a.w))),
+                 fmaxf(fmaxf(fabsf(b.x), fabsf(b.y)), fmaxf(fabsf(b.z), fabsf(b.w))));
+}
+// The exponent of a row whose largest magnitude is mx: the scaled row stays below 2^14.
+__device__ static inline int split_exp(float mx) {
+    if (!(mx > 0.0f && isfinite(mx))) return 0;
+    int k;
+    (void)frexpf(mx, &k);  // mx < 2^k
+    return k - 14;
+}

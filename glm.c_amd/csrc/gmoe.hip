@@ -1056,6 +1056,10 @@ extern "C" int gmoe_forward(gmoe_ctx *c, int layer, int T, const float *x_in, fl
     ra.eps = c->cfg.norm_eps;
     ra.routed_scale = c->cfg.routed_scale;
     ra.force_exact = (flags & GMOE_FLAG_EXACT_ROUTER) != 0;
+    // the grouped GEMMs take xn in split form: from k_rt_dots where that router runs
+    const bool grouped = T >= c->grouped_min_t && !c->native, split_xn = grouped && E <= 64;
+    ra.xspl = split_xn ? c->xspl : nullptr;
+    ra.xexp = c->xexp;
     ProfRecord *pr = prof_begin(c, st, GMOE_KERNEL_ROUTER);
     if (E <= 64) {
         RtParts rp;
@@ -1063,7 +1067,7 @@ extern "C" int gmoe_forward(gmoe_ctx *c, int layer, int T, const float *x_in, fl
         rp.sp = c->rt_sp;
         rp.sa = c->rt_sa;
         hipLaunchKernelGGL(k_rt_norm, dim3((T + 3) / 4), dim3(RT_BLOCK), 0, st, ra, T);
-        hipLaunchKernelGGL(k_rt_dots, dim3((T + 3) / 4, 4), dim3(RT_BLOCK), 0, st, ra, rp, T);
+        hipLaunchKernelGGL(k_rt_dots, dim3((T + 3) / 4, split_xn ? 5 : 4), dim3(RT_BLOCK), 0, st, ra, rp, T);
         hipLaunchKernelGGL(k_rt_select, dim3(T), dim3(RT_BLOCK), 0, st, ra, rp);
     } else {
         hipLaunchKernelGGL(k_router_tok, dim3(T), dim3(RT_BLOCK), 0, st, ra);
@@ -1108,14 +1112,16 @@ extern "C" int gmoe_forward(gmoe_ctx *c, int layer, int T, const float *x_in, fl
             int rc = launch_dispatch(c, T, routed_on, st);
             if (rc) return rc;
         }
-    } else if (T >= c->grouped_min_t) {
+    } else if (grouped) {
         // prefill: digits of xn, the per-expert lists and tiles, grouped gate/up, digits
         // of h, grouped down, per-token combine (grouped.h)
         const int TK = c->Tmax * K;
-        pr = prof_begin(c, st, GMOE_KERNEL_DIGITS);
-        hipLaunchKernelGGL(k_act_split, dim3(T), dim3(GP_BLOCK), 0, st, (const float *)c->xn, D, T, (const int *)nullptr,
-                           c->xspl, c->xexp);
-        prof_end(pr, st);
+        if (!split_xn) {
+            pr = prof_begin(c, st, GMOE_KERNEL_DIGITS);
+            hipLaunchKernelGGL(k_act_split, dim3(T), dim3(GP_BLOCK), 0, st, (const float *)c->xn, D, T, (const int *)nullptr, 0,
+                               c->xspl, c->xexp);
+            prof_end(pr, st);
+        }
         int rc = launch_dispatch(c, T, routed_on, st);
         if (rc) return rc;
         GroupArgs ga;
@@ -1145,11 +1151,9 @@ extern "C" int gmoe_forward(gmoe_ctx *c, int layer, int T, const float *x_in, fl
         prof_end(pr, st);
         // routed rows [0, offsets[E]) and the shared rows [TK, TK + T)
         pr = prof_begin(c, st, GMOE_KERNEL_DIGITS);
-        if (routed_on)
-            hipLaunchKernelGGL(k_act_split, dim3(T * K), dim3(GP_BLOCK), 0, st, (const float *)c->hbuf, F, T * K,
-                               (const int *)(c->offsets + E), c->hspl, c->hexp);
-        hipLaunchKernelGGL(k_act_split, dim3(T), dim3(GP_BLOCK), 0, st, (const float *)(c->hbuf + (size_t)TK * F), F, T,
-                           (const int *)nullptr, c->hspl + (size_t)TK * 2 * F, c->hexp + TK);
+        const int n1 = routed_on ? T * K : 0;
+        hipLaunchKernelGGL(k_act_split, dim3(n1 + T), dim3(GP_BLOCK), 0, st, (const float *)c->hbuf, F, n1,
+                           (const int *)(c->offsets + E), TK, c->hspl, c->hexp);
         prof_end(pr, st);
         ga.aspl = c->hspl;
         ga.aexp = c->hexp;

@@ -37,49 +37,27 @@
 #define GP_BLOCK 256
 #define GP_OCC 3              // blocks per CU the GEMMs are built for (32 KB of LDS each)
 
-// Split form of `rows` rows of n values (n a multiple of 8): sp[r][0][:] = hi and
-// sp[r][1][:] = lo (fp16), ex[r] the exponent. One block per row; rows past *n_rows
-// (when given) are skipped.
-__global__ __launch_bounds__(GP_BLOCK) void k_act_split(const float *__restrict__ v, int n, int rows,
-                                                        const int *__restrict__ n_rows, __half *__restrict__ sp,
+// Split form of rows of n values (n a multiple of 8): sp[r][0][:] = hi and sp[r][1][:] = lo
+// (fp16), ex[r] the exponent. One block per row: block b < n1 takes row b (rows past *n_rows,
+// when given, are skipped), a later one row base2 + b - n1, so that the routed rows and the
+// shared expert's, TK rows on, go in one launch.
+__global__ __launch_bounds__(GP_BLOCK) void k_act_split(const float *__restrict__ v, int n, int n1,
+                                                        const int *__restrict__ n_rows, int base2, __half *__restrict__ sp,
                                                         int *__restrict__ ex) {
     __shared__ float red[GP_BLOCK / 64];
-    const int r = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    if (r >= (n_rows ? *n_rows : rows)) return;
+    const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    if (b < n1 && n_rows && b >= *n_rows) return;
+    const int r = b < n1 ? b : base2 + b - n1;
     const float *src = v + (size_t)r * n;
     float mx = 0.0f;
-    for (int i = tid * 8; i < n; i += GP_BLOCK * 8) {
-        const float4 a = *(const float4 *)(src + i), b = *(const float4 *)(src + i + 4);
-        mx = fmaxf(mx, fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fmaxf(fabsf(a.z), fabsf(a.w))));
-        mx = fmaxf(mx, fmaxf(fmaxf(fabsf(b.x), fabsf(b.y)), fmaxf(fabsf(b.z), fabsf(b.w))));
-    }
+    for (int i = tid * 8; i < n; i += GP_BLOCK * 8) mx = fmaxf(mx, absmax8(src + i));
     mx = wave_max_f(mx);
     if (lane == 0) red[w] = mx;
     __syncthreads();
-    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    int e = 0;
-    if (mx > 0.0f && isfinite(mx)) {
-        int k;
-        (void)frexpf(mx, &k);  // mx < 2^k
-        e = k - 14;            // the scaled row stays below 2^14
-    }
+    const int e = split_exp(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
     if (tid == 0) ex[r] = e;
     __half *hi = sp + (size_t)r * 2 * n, *lo = hi + n;
-    for (int i = tid * 8; i < n; i += GP_BLOCK * 8) {
-        const float4 a = *(const float4 *)(src + i), b = *(const float4 *)(src + i + 4);
-        const float xs[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-        unsigned hw[4], lw[4];  // eight halves of each plane, one 16-byte store each
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const float x0 = ldexpf(xs[2 * k], -e), x1 = ldexpf(xs[2 * k + 1], -e);
-            const __half h0 = __float2half_rn(x0), h1 = __float2half_rn(x1);
-            const __half l0 = __float2half_rn(x0 - __half2float(h0)), l1 = __float2half_rn(x1 - __half2float(h1));
-            hw[k] = (unsigned)__half_as_ushort(h0) | ((unsigned)__half_as_ushort(h1) << 16);
-            lw[k] = (unsigned)__half_as_ushort(l0) | ((unsigned)__half_as_ushort(l1) << 16);
-        }
-        *(uint4 *)(hi + i) = make_uint4(hw[0], hw[1], hw[2], hw[3]);
-        *(uint4 *)(lo + i) = make_uint4(lw[0], lw[1], lw[2], lw[3]);
-    }
+    for (int i = tid * 8; i < n; i += GP_BLOCK * 8) split8(src + i, e, hi + i, lo + i);
 }
 
 struct GroupArgs {

@@ -37,6 +37,8 @@ struct RouterArgs {
     int D, E, K;
     float eps, routed_scale;
     int force_exact;           // GMOE_FLAG_EXACT_ROUTER: skip the certificate, always replay
+    __half *xspl;              // [T][2][D] xn's split form, written by k_rt_dots (null: not wanted)
+    int *xexp;                 // [T]
 };
 
 // (float) of the sequential fp64 mean of squares, decided from a parallel fp64 sum.
@@ -707,8 +709,22 @@ __global__ __launch_bounds__(RT_BLOCK) void k_rt_norm(RouterArgs a, int T) {
 
 #define RT_QMAX (GM_MAX_COLS / 4)  // columns per quarter
 
-// grid (ceil(T/4), 4): wave w takes token 4 blockIdx.x + w, lane e expert e, over the
-// columns of quarter blockIdx.y. The gate rows come through shared memory in tiles of
+// xn of token t in split form (grouped.h), by one wave.
+__device__ __attribute__((always_inline)) static inline void rt_split(const RouterArgs &a, int t, int lane) {
+    const int D = a.D;
+    const float *src = a.xn + (size_t)t * D;
+    float mx = 0.0f;
+    for (int i = 8 * lane; i < D; i += 512) mx = fmaxf(mx, absmax8(src + i));
+    const int e = split_exp(wave_max_f(mx));
+    if (lane == 0) a.xexp[t] = e;
+    __half *hi = a.xspl + (size_t)t * 2 * D, *lo = hi + D;
+    for (int i = 8 * lane; i < D; i += 512) split8(src + i, e, hi + i, lo + i);
+}
+
+// grid (ceil(T/4), 4, or 5 with xn's split form wanted: those blocks write it, a wave per
+// token, beside the dots, which leave most of the chip idle at small T and wait on their own
+// chains at large; a launch of its own takes 5 us there): wave w takes token 4 blockIdx.x + w,
+// lane e expert e, over the columns of quarter blockIdx.y. The gate rows come through shared memory in tiles of
 // 64 columns, [64 experts][16 four-column groups] with group g of row e at slot
 // g ^ (e % 16) (so that the 64 lanes' reads of one group spread over the banks), two
 // tiles in flight; xn's quarter of the block's tokens is staged once.
@@ -719,6 +735,10 @@ __global__ __launch_bounds__(RT_BLOCK) void k_rt_dots(RouterArgs a, RtParts p, i
     const int tg = blockIdx.x, q = blockIdx.y, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int D = a.D, E = a.E, Lq = D / 4, c0 = q * Lq, ntile = Lq / 64;
     const int t = 4 * tg + w;
+    if (q == 4) {
+        if (t < T) rt_split(a, t, lane);
+        return;
+    }
     // The quarters by DMA too, issued first: Lq pieces of 16 bytes (Lq / 4 a row), 64 to a
     // wave's DMA, dealt round the waves. A token past T reads token T - 1 (its sums are not stored).
     for (int s = w; s < Lq / 64; s += 4) {
