@@ -325,20 +325,30 @@ __device__ static inline float digits_to_float(int D0, int D1, int D2) {
 
 // ---------------------------------------------------------------- split activations
 //
-// Columns i .. i + 7 of a row of fp32 values in the GEMMs' split form: hi = fp16(v 2^-e) and
-// lo = fp16(v 2^-e - hi), one 16-byte store each.
-__device__ static inline void split8(const float *src, int e, __half *hi, __half *lo) {
-    const float4 a = *(const float4 *)src, b = *(const float4 *)(src + 4);
-    const float xs[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    unsigned hw[4], lw[4];
+// Four consecutive values of a row in the GEMMs' split form: hi = fp16(v 2^-e) and lo =
+// fp16(v 2^-e - hi), as two dwords each; split4 stores them, split8 eight in 16-byte stores.
+__device__ static inline void split_pack(const float *xs, int e, unsigned *hw, unsigned *lw) {
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
+    for (int k = 0; k < 2; k++) {
         const float x0 = ldexpf(xs[2 * k], -e), x1 = ldexpf(xs[2 * k + 1], -e);
         const __half h0 = __float2half_rn(x0), h1 = __float2half_rn(x1);
         const __half l0 = __float2half_rn(x0 - __half2float(h0)), l1 = __float2half_rn(x1 - __half2float(h1));
         hw[k] = (unsigned)__half_as_ushort(h0) | ((unsigned)__half_as_ushort(h1) << 16);
         lw[k] = (unsigned)__half_as_ushort(l0) | ((unsigned)__half_as_ushort(l1) << 16);
     }
+}
+__device__ static inline void split4(const float *v, int e, __half *hi, __half *lo) {
+    unsigned hw[2], lw[2];
+    split_pack(v, e, hw, lw);
+    *(uint2 *)hi = make_uint2(hw[0], hw[1]);
+    *(uint2 *)lo = make_uint2(lw[0], lw[1]);
+}
+__device__ static inline void split8(const float *src, int e, __half *hi, __half *lo) {
+    const float4 a = *(const float4 *)src, b = *(const float4 *)(src + 4);
+    const float xs[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    unsigned hw[4], lw[4];
+    split_pack(xs, e, hw, lw);
+    split_pack(xs + 4, e, hw + 2, lw + 2);
     *(uint4 *)hi = make_uint4(hw[0], hw[1], hw[2], hw[3]);
     *(uint4 *)lo = make_uint4(lw[0], lw[1], lw[2], lw[3]);
 }

@@ -2,10 +2,10 @@
 //
 // A decode call (T=1) is one persistent launch, k_moe_stack (stack.h), that takes
 // the token through any run of layers. A batch (T>1) runs per layer:
-//   k_rt_norm       grid (T/4)             rmsnorm, a wave per token (router.h; E <= 64, else k_router_tok does all three)
-//   k_rt_dots       grid (T/4, 4)          router logits' sums, a thread per (token, expert, quarter of D)
+//   k_rt_dots       grid (T/4, 5)          rmsnorm and the router logits' sums, a thread per (token, expert, quarter of
+//                                          D); the fifth row writes xn, and as fp16 hi+lo planes with a per-row
+//                                          exponent (grouped.h) (router.h; E <= 64, else k_router_tok does it all)
 //   k_rt_select     grid (T)               bounds, certified top-k, exact replay when needed
-//   k_act_split     grid (rows)            xn as fp16 hi+lo planes with a per-row exponent (grouped.h)
 //   k_dispatch      grid (E)               exact per-expert token lists and GEMM tiles (dispatch.h)
 //   k_group_gu      grid (F/64, tiles)     grouped gate/up GEMM + SwiGLU on fp16 MFMA (grouped.h)
 //   k_act_split     grid (rows)            h as fp16 hi+lo planes
@@ -1066,8 +1066,7 @@ extern "C" int gmoe_forward(gmoe_ctx *c, int layer, int T, const float *x_in, fl
         rp.t = c->rt_t;
         rp.sp = c->rt_sp;
         rp.sa = c->rt_sa;
-        hipLaunchKernelGGL(k_rt_norm, dim3((T + 3) / 4), dim3(RT_BLOCK), 0, st, ra, T);
-        hipLaunchKernelGGL(k_rt_dots, dim3((T + 3) / 4, split_xn ? 5 : 4), dim3(RT_BLOCK), 0, st, ra, rp, T);
+        hipLaunchKernelGGL(k_rt_dots, dim3((T + 3) / 4, 5), dim3(RT_BLOCK), 0, st, ra, rp, T);
         hipLaunchKernelGGL(k_rt_select, dim3(T), dim3(RT_BLOCK), 0, st, ra, rp);
     } else {
         hipLaunchKernelGGL(k_router_tok, dim3(T), dim3(RT_BLOCK), 0, st, ra);

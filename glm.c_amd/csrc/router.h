@@ -37,7 +37,7 @@ struct RouterArgs {
     int D, E, K;
     float eps, routed_scale;
     int force_exact;           // GMOE_FLAG_EXACT_ROUTER: skip the certificate, always replay
-    __half *xspl;              // [T][2][D] xn's split form, written by k_rt_dots (null: not wanted)
+    __half *xspl;              // [T][2][D] xn's split form, for k_rt_dots to write (null: not wanted)
     int *xexp;                 // [T]
 };
 
@@ -641,10 +641,10 @@ __global__ __launch_bounds__(RT_BLOCK) void k_router_tok(RouterArgs a) {
     for (int i = tid; i < E; i += RT_BLOCK) a.router_prob[(size_t)t * E + i] = s_p[i];
 }
 
-// ---------------------------------------------------------------- the router of T > 1, in three kernels
+// ---------------------------------------------------------------- the router of T > 1, in two kernels
 //
-// For E <= 64 the router of a batch runs as k_rt_norm (rmsnorm, one block per token),
-// k_rt_dots (the logits' sums) and k_rt_select (bounds, certified top-k, exact replay),
+// For E <= 64 the router of a batch runs as k_rt_dots (rmsnorm and the logits' sums) and
+// k_rt_select (bounds, certified top-k, exact replay),
 // rather than k_router_tok's one block per token: there, each expert's dot is a
 // wave-wide reduction, and its fp64 scans and sums leave the SIMDs issue-bound.
 // k_rt_dots gives every (token, expert, quarter of D) its own thread, which runs the
@@ -659,75 +659,98 @@ struct RtParts {
     float *sa;   // [T][4][E] quarter sums of |g x| (fp32)
 };
 
-// grid (ceil(T/4)): xn of token 4 blockIdx.x + w on wave w (infer.c:746-752),
-// bit-identical to glm.c: lane l holds the row's D/64 consecutive values from l D/64, the
-// mean of squares is certified from the wave's fp64 sum (relative error below D 2^-52)
-// or else replayed in order by lane 0, and xn is formed from the registers.
-__global__ __launch_bounds__(RT_BLOCK) void k_rt_norm(RouterArgs a, int T) {
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, t = 4 * blockIdx.x + w, D = a.D;
-    if (t >= T) return;  // wave-uniform
-    const int per = D / 64;  // a multiple of 4, at most RT_CPL_MAX
-    const float *xt = a.x + (size_t)t * D;
+// Token t's row on one wave (infer.c:746-752): lane l's D/64 consecutive values from l D/64
+// into xv, and the rmsnorm's factor, bit-identical to glm.c: the mean of squares is certified
+// from the wave's fp64 sum (relative error below D 2^-52) or else replayed in order by lane 0
+// (counted where `count` says so: several blocks norm the same token).
+struct RtRow {
     float xv[RT_CPL_MAX];
+};
+__device__ __attribute__((always_inline)) static inline void rt_row_load(const RouterArgs &a, int t, int lane, RtRow &r) {
+    const int per = a.D / 64;  // a multiple of 4, at most RT_CPL_MAX
+    const float *xt = a.x + (size_t)t * a.D;
     if (((uintptr_t)a.x & 15) == 0) {  // the caller's x: 16-byte loads when aligned
 #pragma unroll
         for (int q = 0; q < RT_CPL_MAX / 4; q++) {
             const float4 v = q < per / 4 ? *(const float4 *)(xt + lane * per + 4 * q) : make_float4(0.f, 0.f, 0.f, 0.f);
-            xv[4 * q] = v.x;
-            xv[4 * q + 1] = v.y;
-            xv[4 * q + 2] = v.z;
-            xv[4 * q + 3] = v.w;
+            r.xv[4 * q] = v.x;
+            r.xv[4 * q + 1] = v.y;
+            r.xv[4 * q + 2] = v.z;
+            r.xv[4 * q + 3] = v.w;
         }
     } else {
 #pragma unroll
-        for (int j = 0; j < RT_CPL_MAX; j++) xv[j] = j < per ? xt[lane * per + j] : 0.0f;
+        for (int j = 0; j < RT_CPL_MAX; j++) r.xv[j] = j < per ? xt[lane * per + j] : 0.0f;
     }
+}
+__device__ __attribute__((always_inline)) static inline float rt_row_inv(const RouterArgs &a, int t, int lane, const RtRow &r,
+                                                                        bool count) {
+    const int D = a.D;
     double ss = 0.0;
 #pragma unroll
-    for (int j = 0; j < RT_CPL_MAX; j++) ss += (double)xv[j] * (double)xv[j];
+    for (int j = 0; j < RT_CPL_MAX; j++) ss += (double)r.xv[j] * (double)r.xv[j];
     ss = wave_sum_dpp(ss);
     const double v = ss / (double)D, rho = (double)D * 0x1p-52;
     float mean = (float)(v * (1.0 - rho));
     if (mean != (float)(v * (1.0 + rho))) {  // wave-uniform
+        const float *xt = a.x + (size_t)t * D;
         double sq = 0.0;
         if (lane == 0) {
             for (int i = 0; i < D; i++) sq += (double)xt[i] * (double)xt[i];
-            atomicAdd(&a.stats[GM_STAT_NORM_EXACT], 1ull);
+            if (count) atomicAdd(&a.stats[GM_STAT_NORM_EXACT], 1ull);
         }
         mean = (float)(readlane_d(sq, 0) / (double)D);
     }
-    const float inv = __fdiv_rn(1.0f, sqrt_rn_f32(__fadd_rn(mean, a.eps)));
+    return __fdiv_rn(1.0f, sqrt_rn_f32(__fadd_rn(mean, a.eps)));
+}
+// The row's xn in place of its x.
+__device__ __attribute__((always_inline)) static inline void rt_row_xn(const RouterArgs &a, int lane, float inv, RtRow &r) {
+    const int per = a.D / 64;
 #pragma unroll
     for (int q = 0; q < RT_CPL_MAX / 4; q++)
         if (q < per / 4) {
             const float4 nw = *(const float4 *)(a.norm_w + lane * per + 4 * q);
-            *(float4 *)(a.xn + (size_t)t * D + lane * per + 4 * q) =
-                make_float4(__fmul_rn(__fmul_rn(xv[4 * q], inv), nw.x), __fmul_rn(__fmul_rn(xv[4 * q + 1], inv), nw.y),
-                            __fmul_rn(__fmul_rn(xv[4 * q + 2], inv), nw.z), __fmul_rn(__fmul_rn(xv[4 * q + 3], inv), nw.w));
+            const float w[4] = {nw.x, nw.y, nw.z, nw.w};
+#pragma unroll
+            for (int c = 0; c < 4; c++) r.xv[4 * q + c] = __fmul_rn(__fmul_rn(r.xv[4 * q + c], inv), w[c]);
         }
 }
 
 #define RT_QMAX (GM_MAX_COLS / 4)  // columns per quarter
 
-// xn of token t in split form (grouped.h), by one wave.
-__device__ __attribute__((always_inline)) static inline void rt_split(const RouterArgs &a, int t, int lane) {
-    const int D = a.D;
-    const float *src = a.xn + (size_t)t * D;
+// xn of token t to memory and, where wanted, its split form (grouped.h), by one wave.
+__device__ __attribute__((always_inline)) static inline void rt_xn_store(const RouterArgs &a, int t, int lane) {
+    const int D = a.D, per = D / 64;
+    RtRow r;
+    rt_row_load(a, t, lane, r);
+    rt_row_xn(a, lane, rt_row_inv(a, t, lane, r, true), r);
+    float *xn = a.xn + (size_t)t * D + lane * per;
     float mx = 0.0f;
-    for (int i = 8 * lane; i < D; i += 512) mx = fmaxf(mx, absmax8(src + i));
+#pragma unroll
+    for (int q = 0; q < RT_CPL_MAX / 4; q++)
+        if (q < per / 4) {
+            const float *v = r.xv + 4 * q;
+            *(float4 *)(xn + 4 * q) = make_float4(v[0], v[1], v[2], v[3]);
+            mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
+        }
+    if (!a.xspl) return;
     const int e = split_exp(wave_max_f(mx));
     if (lane == 0) a.xexp[t] = e;
-    __half *hi = a.xspl + (size_t)t * 2 * D, *lo = hi + D;
-    for (int i = 8 * lane; i < D; i += 512) split8(src + i, e, hi + i, lo + i);
+    __half *hi = a.xspl + (size_t)t * 2 * D + lane * per, *lo = hi + D;
+#pragma unroll
+    for (int q = 0; q < RT_CPL_MAX / 4; q++)
+        if (q < per / 4) split4(r.xv + 4 * q, e, hi + 4 * q, lo + 4 * q);
 }
 
-// grid (ceil(T/4), 4, or 5 with xn's split form wanted: those blocks write it, a wave per
-// token, beside the dots, which leave most of the chip idle at small T and wait on their own
-// chains at large; a launch of its own takes 5 us there): wave w takes token 4 blockIdx.x + w,
-// lane e expert e, over the columns of quarter blockIdx.y. The gate rows come through shared memory in tiles of
+// grid (ceil(T/4), 5): wave w takes token 4 blockIdx.x + w. Blocks 0..3 of a row: lane e
+// expert e, over the columns of quarter blockIdx.y; block 4: xn and its split form to memory.
+// Each forms the rmsnorm for itself (8 KB of x a token, from L2, while the first gate tiles
+// come in) rather than a launch before this one: 5 to 6 us of a small batch's layer (8 tokens:
+// 98 -> 92 us).
+// The gate rows come through shared memory in tiles of
 // 64 columns, [64 experts][16 four-column groups] with group g of row e at slot
 // g ^ (e % 16) (so that the 64 lanes' reads of one group spread over the banks), two
-// tiles in flight; xn's quarter of the block's tokens is staged once.
+// tiles in flight; a wave's quarter of xn lies there too.
 #define RT_DOT_STAGES 3  // router-row tiles in shared memory: two in flight while one is used
 __global__ __launch_bounds__(RT_BLOCK) void k_rt_dots(RouterArgs a, RtParts p, int T) {
     __shared__ __align__(16) float4 gt[RT_DOT_STAGES][64 * 16];
@@ -736,16 +759,11 @@ __global__ __launch_bounds__(RT_BLOCK) void k_rt_dots(RouterArgs a, RtParts p, i
     const int D = a.D, E = a.E, Lq = D / 4, c0 = q * Lq, ntile = Lq / 64;
     const int t = 4 * tg + w;
     if (q == 4) {
-        if (t < T) rt_split(a, t, lane);
+        if (t < T) rt_xn_store(a, t, lane);
         return;
     }
-    // The quarters by DMA too, issued first: Lq pieces of 16 bytes (Lq / 4 a row), 64 to a
-    // wave's DMA, dealt round the waves. A token past T reads token T - 1 (its sums are not stored).
-    for (int s = w; s < Lq / 64; s += 4) {
-        const int piece = 64 * s + lane, tw = piece / (Lq / 4), k = 4 * (piece - tw * (Lq / 4));
-        const int tt = min(4 * tg + tw, T - 1);
-        dma16_untracked(gbl(a.xn + (size_t)tt * D + c0 + k), (lds_void *)(xs + 256 * s));
-    }
+    RtRow row;  // a token past T takes token T - 1 (its sums are not stored)
+    rt_row_load(a, min(t, T - 1), lane, row);
     auto stage = [&](int j, int buf) {  // 1024 pieces of 16 bytes: four per lane
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -754,17 +772,28 @@ __global__ __launch_bounds__(RT_BLOCK) void k_rt_dots(RouterArgs a, RtParts p, i
             dma16_untracked(gbl(a.gate_inp + (size_t)ee * D + c0 + 64 * j + 4 * g), (lds_void *)(gt[buf] + (4 * w + i) * 64));
         }
     };
-    // tiles of 64 columns, two ahead. Each stage() is four DMAs a thread; the waits below
-    // count them in order, so vmcnt(4) after stage(1) also covers the quarters' DMAs.
-    // The barriers are s_barrier in inline assembly after an exact wait (with the shared-memory
-    // stores and reads done): __syncthreads() would also wait for the DMAs still in flight.
+    // tiles of 64 columns, two ahead. Each stage() is four DMAs a thread, counted in order by
+    // the waits below. The barriers are s_barrier in inline assembly after an exact wait (with
+    // the shared-memory stores and reads done): __syncthreads() would also wait for the DMAs
+    // still in flight.
     stage(0, 0);
-    if (ntile > 1) {
-        stage(1, 1);
-        asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    } else {
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (ntile > 1) stage(1, 1);
+    {
+        const float inv = rt_row_inv(a, min(t, T - 1), lane, row, false);
+        const int per = D / 64;
+        if ((lane >> 4) == q) {  // the lanes that hold the quarter's columns
+            rt_row_xn(a, lane, inv, row);
+#pragma unroll
+            for (int k = 0; k < RT_CPL_MAX / 4; k++)
+                if (k < per / 4)
+                    *(float4 *)(xs + w * Lq + (lane & 15) * per + 4 * k) =
+                        make_float4(row.xv[4 * k], row.xv[4 * k + 1], row.xv[4 * k + 2], row.xv[4 * k + 3]);
+        }
     }
+    if (ntile > 1)
+        asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    else
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     double acc = 0.0, sp = 0.0;
     float sa = 0.0f;
     for (int j = 0; j < ntile; j++) {
