@@ -12,8 +12,10 @@
 //   k_group_down    grid (D/64, tiles)     grouped down GEMM, one row per (token, slot) (grouped.h)
 //   k_token_combine grid (D/1024, T)       weighted combine + shared expert + residual (grouped.h)
 // With GMOE_GROUPED_MIN_T above T, batches take the per-token kernels k_gate_up and
-// k_down_combine (experts.h) instead. Expert weights are uploaded once per layer
-// into the tiled Q8_0 layout of common.h and stay resident.
+// k_down_combine (experts.h) instead. Experts in glm.c's own layout take k_native_group_gu and
+// k_native_group_down in the GEMMs' place, and at small batches native.h's per-token kernels.
+// Expert weights are uploaded once per layer into the tiled Q8_0 layout of common.h (or, in
+// the native form, as they are) and stay resident.
 #include "gmoe.h"
 
 #include <gnu/libc-version.h>
@@ -1015,6 +1017,20 @@ static int check_stack_error(gmoe_ctx *c) {
     return GMOE_OK;
 }
 
+// The native form's grouped GEMM (gate/up or down) for NS scales per chunk.
+static void launch_native_group(int ns, bool gu, dim3 grid, const GroupArgs &ga, hipStream_t st) {
+    const dim3 block(GP_BLOCK);
+    if (gu) {
+        if (ns == 2) hipLaunchKernelGGL(k_native_group_gu<2>, grid, block, 0, st, ga);
+        else if (ns == 4) hipLaunchKernelGGL(k_native_group_gu<4>, grid, block, 0, st, ga);
+        else hipLaunchKernelGGL(k_native_group_gu<8>, grid, block, 0, st, ga);
+    } else {
+        if (ns == 2) hipLaunchKernelGGL(k_native_group_down<2>, grid, block, 0, st, ga);
+        else if (ns == 4) hipLaunchKernelGGL(k_native_group_down<4>, grid, block, 0, st, ga);
+        else hipLaunchKernelGGL(k_native_group_down<8>, grid, block, 0, st, ga);
+    }
+}
+
 extern "C" int gmoe_forward(gmoe_ctx *c, int layer, int T, const float *x_in, float *x_out, int flags,
                             void *stream) {
     if (!c || !x_in || !x_out) {
@@ -1056,8 +1072,14 @@ extern "C" int gmoe_forward(gmoe_ctx *c, int layer, int T, const float *x_in, fl
     ra.eps = c->cfg.norm_eps;
     ra.routed_scale = c->cfg.routed_scale;
     ra.force_exact = (flags & GMOE_FLAG_EXACT_ROUTER) != 0;
+    // The native form's per-token kernels read T (K + 1) experts, its grouped GEMMs those touched
+    // plus three launches more. Two layers at D 2048, F 1536, group size 64, per-token against
+    // grouped: E 64, K 4: 284 / 290 us at T = 12, 351 / 320 at 16; E 32, K 8: 205 / 228 at 4,
+    // 270 / 246 at 6; E 128, K 8: 478 / 499 at 9, 703 / 628 at 16; E 32, K 2: 145 / 171 at 8,
+    // 225 / 192 at 16. The line T (K + 1) = E + 2 K lies past each crossing.
+    const bool grouped = T >= c->grouped_min_t && (!c->native || T * (K + 1) >= E + 2 * K);
     // the grouped GEMMs take xn in split form: from k_rt_dots where that router runs
-    const bool grouped = T >= c->grouped_min_t && !c->native, split_xn = grouped && E <= 64;
+    const bool split_xn = grouped && E <= 64;
     ra.xspl = split_xn ? c->xspl : nullptr;
     ra.xexp = c->xexp;
     ProfRecord *pr = prof_begin(c, st, GMOE_KERNEL_ROUTER);
@@ -1074,7 +1096,7 @@ extern "C" int gmoe_forward(gmoe_ctx *c, int layer, int T, const float *x_in, fl
     prof_end(pr, st);
     const int routed_on = !(fl & GMOE_FLAG_NO_ROUTED);
     c->last_dispatched = 0;
-    if (c->native) {
+    if (c->native && !grouped) {
         // checkpoint-layout experts (native.h): gate/up + SwiGLU, down, combine; the
         // per-expert lists for T > 1 as on the other paths
         NativeArgs na;
@@ -1116,7 +1138,8 @@ extern "C" int gmoe_forward(gmoe_ctx *c, int layer, int T, const float *x_in, fl
         // of h, grouped down, per-token combine (grouped.h)
         const int TK = c->Tmax * K;
         if (!split_xn) {
-            pr = prof_begin(c, st, GMOE_KERNEL_DIGITS);
+            // (the native form has no entry of its own for these: counted with the product they feed)
+            pr = prof_begin(c, st, c->native ? GMOE_KERNEL_GATE_UP : GMOE_KERNEL_DIGITS);
             hipLaunchKernelGGL(k_act_split, dim3(T), dim3(GP_BLOCK), 0, st, (const float *)c->xn, D, T, (const int *)nullptr, 0,
                                c->xspl, c->xexp);
             prof_end(pr, st);
@@ -1143,13 +1166,16 @@ extern "C" int gmoe_forward(gmoe_ctx *c, int layer, int T, const float *x_in, fl
         ga.aspl = c->xspl;
         ga.aexp = c->xexp;
         ga.out = c->hbuf;
+        ga.gs_inv = c->native ? gn_inv(c->cfg.group_size) : 0;
+        const int ns = c->native ? gn_scales(c->cfg.group_size) : 0;
         const int max_tiles = (routed_on ? E + (T * K + GP_TOK - 1) / GP_TOK : 0) + (T + GP_TOK - 1) / GP_TOK;
         pr = prof_begin(c, st, GMOE_KERNEL_GATE_UP);
-        if (c->g16) hipLaunchKernelGGL(k_group_gu<true>, dim3(F / 64, max_tiles), dim3(GP_BLOCK), 0, st, ga);
+        if (ns) launch_native_group(ns, true, dim3(F / 64, max_tiles), ga, st);
+        else if (c->g16) hipLaunchKernelGGL(k_group_gu<true>, dim3(F / 64, max_tiles), dim3(GP_BLOCK), 0, st, ga);
         else hipLaunchKernelGGL(k_group_gu<false>, dim3(F / 64, max_tiles), dim3(GP_BLOCK), 0, st, ga);
         prof_end(pr, st);
         // routed rows [0, offsets[E]) and the shared rows [TK, TK + T)
-        pr = prof_begin(c, st, GMOE_KERNEL_DIGITS);
+        pr = prof_begin(c, st, c->native ? GMOE_KERNEL_DOWN : GMOE_KERNEL_DIGITS);
         const int n1 = routed_on ? T * K : 0;
         hipLaunchKernelGGL(k_act_split, dim3(n1 + T), dim3(GP_BLOCK), 0, st, (const float *)c->hbuf, F, n1,
                            (const int *)(c->offsets + E), TK, c->hspl, c->hexp);
@@ -1158,7 +1184,8 @@ extern "C" int gmoe_forward(gmoe_ctx *c, int layer, int T, const float *x_in, fl
         ga.aexp = c->hexp;
         ga.out = c->ybuf;
         pr = prof_begin(c, st, GMOE_KERNEL_DOWN);
-        if (c->g16) hipLaunchKernelGGL(k_group_down<true>, dim3(D / 64, max_tiles), dim3(GP_BLOCK), 0, st, ga);
+        if (ns) launch_native_group(ns, false, dim3(D / 64, max_tiles), ga, st);
+        else if (c->g16) hipLaunchKernelGGL(k_group_down<true>, dim3(D / 64, max_tiles), dim3(GP_BLOCK), 0, st, ga);
         else hipLaunchKernelGGL(k_group_down<false>, dim3(D / 64, max_tiles), dim3(GP_BLOCK), 0, st, ga);
         prof_end(pr, st);
         TokenCombineArgs ta;

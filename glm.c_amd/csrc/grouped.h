@@ -70,6 +70,7 @@ struct GroupArgs {
     const __half *aspl;      // activations split: [token or list row][2 (hi, lo)][cols]
     const int *aexp;
     float *out;              // [TK + T][cols out] per list row
+    unsigned gs_inv;         // native form: gn_inv(group size)
 };
 
 // Token (for the gate/up input) of list row `row`.
@@ -122,13 +123,15 @@ __device__ static inline void gp_stage(const GpStage<NA> &g, uint8_t *buf, int c
 }
 
 // The A operand of A tile i (inputs 16i..16i+15), plane pl, for 32-column block b of
-// the staged chunk: lane l holds input 16i + l % 16, columns 32b + 8(l / 16) .. +8.
-__device__ static inline gp_h8 gp_a(const uint8_t *buf, int i, int pl, int b) {
+// the staged chunk: lane l holds input 16i + l % 16, columns 32b + 8u .. +8 with u = l / 16 (or
+// as the B operand's lane order has it).
+__device__ static inline gp_h8 gp_a(const uint8_t *buf, int i, int pl, int b, int u) {
     const int lane = threadIdx.x & 63;
     const int in = 16 * i + (lane & 15), r = 2 * in + pl;
-    const int j = 4 * b + (lane >> 4), p = j ^ (in & 15);
+    const int j = 4 * b + u, p = j ^ (in & 15);
     return *(const gp_h8 *)(buf + r * GP_RB + 16 * p);
 }
+__device__ static inline gp_h8 gp_a(const uint8_t *buf, int i, int pl, int b) { return gp_a(buf, i, pl, b, (threadIdx.x & 63) >> 4); }
 
 // Eight int8 weights (two dwords) as fp16, exactly: each byte b becomes the fp16 with
 // bits 0x64 (b ^ 0x80) = 1152 + q, and one packed subtract removes the 1152.
@@ -444,6 +447,215 @@ __global__ __launch_bounds__(GP_BLOCK, GP_OCC) void k_group_down(GroupArgs a) {
     const GpTile tl = a.tiles[blockIdx.y];
     gp_with_na<GP_NA_MAX>(__builtin_amdgcn_readfirstlane((tl.count + 15) >> 4),
                           [&](auto NA) { gp_down_tile<decltype(NA)::value, G16>(a, tl, abuf); });
+}
+
+// ---- the native form (native.h: glm.c's rows of int8 and fp32 scales, any group size) -------
+//
+// The same tiles and activations as above over weights in glm.c's own layout. A lane reads 16
+// consecutive bytes of its row per 64-column piece (lane l: row l % 16, columns 16 (l / 16) ..),
+// so that four lanes read a row's piece as one 64-byte run, and two exchanges between the wave's
+// halves (v_permlane32_swap) bring the piece's first and second 32 columns together as two B
+// operands, whose lane l / 16 then holds the 8-column units 0, 2, 1, 3 of its block.
+// NS: fp32 scales a row has per chunk of GP_KC = 128 columns: 2 (group size a multiple of 64:
+// a piece's four MFMAs share one scale), 4 (of 32) or 8 (of 16: a block's halves apart).
+// Weights are read once per tile of 32 tokens where k_native_gate_up and k_native_down
+// (native.h, kept for T = 1) read them once per token and slot.
+__host__ __device__ constexpr int gn_scales(int gs) { return gs % 64 == 0 ? 2 : gs % 32 == 0 ? 4 : 8; }
+// Group of the 16-column unit u (of a row of at most 2048 columns): u / (gs / 16) as a product.
+__host__ __device__ constexpr unsigned gn_inv(int gs) { return 65536u / (unsigned)(gs / 16) + 1; }
+__host__ __device__ constexpr unsigned gn_group(unsigned u, unsigned inv) { return u * inv >> 16; }
+constexpr bool gn_group_exact() {
+    for (unsigned g = 1; g <= GM_MAX_COLS / 16; g++)
+        for (unsigned u = 0; u < GM_MAX_COLS / 16; u++)
+            if (gn_group(u, gn_inv(16 * (int)g)) != u / g) return false;
+    return true;
+}
+static_assert(gn_group_exact(), "the product is the division for every group size and unit");
+
+template <int NM, int NS>
+struct GnRegs {
+    u32x4 q[NM][GP_NB / 2];
+    float s[NM][NS];
+};
+__host__ __device__ constexpr int gn_loads(int na, int nm, int ns) { return nm * (GP_NB / 2 + ns) + gp_stage_iters(na); }
+
+// The tile's products with rows 64 blockIdx.x .. of NM matrices (q planes at qm[], scales at
+// sm[], `cols` columns): store(i, k, row, sums) per input 16i + 4(l/16) + k of the lane's row.
+template <int NA, int NM, int NS, typename RowOf, typename Store>
+__device__ __attribute__((always_inline)) static inline void gn_tile(const GroupArgs &a, int cols, const uint8_t *const (&qm)[NM],
+                                                                     const uint8_t *const (&sm)[NM], RowOf src_row, Store store,
+                                                                     gp_abuf3_t &abuf) {
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, qh = lane >> 4;
+    const int row = 64 * blockIdx.x + 16 * w + (lane & 15);
+    const int unit = 2 * (qh & 1) + (qh >> 1);  // the lane's 8-column unit of a block
+    const unsigned inv = a.gs_inv;
+    const int ng = gn_group(cols / 16 - 1, inv) + 1;
+    const GM_GLOBAL u32x4 *q[NM];
+    const GM_GLOBAL float *sc[NM];
+#pragma unroll
+    for (int m = 0; m < NM; m++) {
+        q[m] = gbl((const u32x4 *)(qm[m] + (size_t)row * cols)) + qh;
+        sc[m] = gbl((const float *)sm[m] + (size_t)row * ng);
+    }
+    const GpStage<NA> stg = gp_stage_init<NA>(a.aspl, cols, src_row);
+    const int nkc = cols / GP_KC;
+    float acc[NM][NA][4];
+#pragma unroll
+    for (int m = 0; m < NM; m++)
+#pragma unroll
+        for (int i = 0; i < NA; i++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) acc[m][i][k] = 0.0f;
+    auto issue = [&](GnRegs<NM, NS> &r, int kc) {  // gn_loads(NA, NM, NS) loads
+#pragma unroll
+        for (int m = 0; m < NM; m++)
+#pragma unroll
+            for (int u = 0; u < GP_NB / 2; u++) r.q[m][u] = q[m][4 * ((GP_NB / 2) * kc + u)];
+#pragma unroll
+        for (int m = 0; m < NM; m++)
+#pragma unroll
+            for (int j = 0; j < NS; j++) r.s[m][j] = sc[m][gn_group((GP_KC / 16) * kc + (GP_KC / 16) / NS * j, inv)];
+        gp_stage<NA>(stg, abuf[kc % 3], kc * GP_KC);
+    };
+    // A chunk's products are summed apart before they join the running sum, and the first half of
+    // the chunks apart from the second: with every block added to one running sum the roundings
+    // at its size made a layer 2.7e-7 from 64 bits where the per-token kernels' fp32 tree is
+    // 2.21e-7 to 2.25e-7 (D 2048, F 1536, group size 64); so it is 2.15e-7 to 2.2e-7.
+    auto compute = [&](const GnRegs<NM, NS> &r, int kc) {
+        const uint8_t *buf = abuf[kc % 3];
+#pragma unroll
+        for (int m = 0; m < NM; m++) {
+            // (the second matrix reads the inputs again: kept from the first, they cost 64 registers)
+            if (m) asm volatile("" ::: "memory");
+            float t[NA][4];
+            auto add = [&](int i, gp_f4 d, float s, bool first) {
+#pragma unroll
+                for (int k = 0; k < 4; k++) t[i][k] = first ? __fmul_rn(d[k], s) : fmaf(d[k], s, t[i][k]);
+            };
+#pragma unroll
+            for (int u = 0; u < GP_NB / 2; u++) {
+                typedef unsigned u2 __attribute__((ext_vector_type(2)));
+                const u32x4 c = r.q[m][u];
+                const u2 xz = __builtin_amdgcn_permlane32_swap(c.x, c.z, false, false);
+                const u2 yw = __builtin_amdgcn_permlane32_swap(c.y, c.w, false, false);
+                const gp_h8 B[2] = {gp_i8_to_h8(xz[0], yw[0]), gp_i8_to_h8(xz[1], yw[1])};
+                const gp_f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+                if constexpr (NS == 2) {
+#pragma unroll
+                    for (int i = 0; i < NA; i++) {
+                        gp_f4 d = zero;  // the small lo products first
+#pragma unroll
+                        for (int pl = 1; pl >= 0; pl--)
+#pragma unroll
+                            for (int b = 0; b < 2; b++)
+                                d = __builtin_amdgcn_mfma_f32_16x16x32_f16(gp_a(buf, i, pl, 2 * u + b, unit), B[b], d, 0, 0, 0);
+                        add(i, d, r.s[m][u], u == 0);
+                    }
+                } else {
+                    constexpr int H = NS / 4;  // scales a block
+#pragma unroll
+                    for (int b = 0; b < 2; b++)
+#pragma unroll
+                        for (int h = 0; h < H; h++) {
+                            const gp_h8 none = {};
+                            const gp_h8 Bh = H == 1 || (qh & 1) == h ? B[b] : none;  // units 0, 1 or 2, 3
+#pragma unroll
+                            for (int i = 0; i < NA; i++) {
+                                gp_f4 d = __builtin_amdgcn_mfma_f32_16x16x32_f16(gp_a(buf, i, 1, 2 * u + b, unit), Bh, zero, 0, 0, 0);
+                                d = __builtin_amdgcn_mfma_f32_16x16x32_f16(gp_a(buf, i, 0, 2 * u + b, unit), Bh, d, 0, 0, 0);
+                                add(i, d, r.s[m][H * (2 * u + b) + h], u == 0 && b == 0 && h == 0);
+                            }
+                        }
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < NA; i++)
+#pragma unroll
+                for (int k = 0; k < 4; k++) acc[m][i][k] = __fadd_rn(acc[m][i][k], t[i][k]);
+        }
+    };
+    auto step = [&](GnRegs<NM, NS> &r, GnRegs<NM, NS> &rn, int kc) {  // as k_group_gu's
+        if (kc + 2 < nkc) {
+            issue(rn, kc + 2);
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * gn_loads(NA, NM, NS)) : "memory");
+        } else if (kc + 1 < nkc) {
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(gn_loads(NA, NM, NS)) : "memory");
+        } else {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
+        gp_barrier();
+        compute(r, kc);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        gp_barrier();
+    };
+    static_assert(2 * gn_loads(GP_NA_MAX, 2, 8) < 64, "vmcnt counts six bits");
+    float first[NM][NA][4];  // the first half of the chunks
+    const int mid = (nkc + 5) / 6 * 3;
+    GnRegs<NM, NS> r0, r1, r2;
+    issue(r0, 0);
+    if (nkc > 1) issue(r1, 1);
+    for (int kc = 0; kc < nkc; kc += 3) {
+        if (kc == 0 || kc == mid) {
+#pragma unroll
+            for (int m = 0; m < NM; m++)
+#pragma unroll
+                for (int i = 0; i < NA; i++)
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        first[m][i][k] = acc[m][i][k];
+                        acc[m][i][k] = 0.0f;
+                    }
+        }
+        step(r0, r2, kc);
+        if (kc + 1 < nkc) step(r1, r0, kc + 1);
+        if (kc + 2 < nkc) step(r2, r1, kc + 2);
+    }
+#pragma unroll
+    for (int i = 0; i < NA; i++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            float v[NM];
+#pragma unroll
+            for (int m = 0; m < NM; m++) v[m] = __fadd_rn(first[m][i][k], acc[m][i][k]);
+            store(16 * i + 4 * qh + k, row, v);
+        }
+}
+
+// k_group_gu and k_group_down over the native form (same grids and outputs). 64 tokens, D 2048,
+// F 1536, 64 experts, group size 64: 134 and 72 us (4.9 and 4.5 TB/s of the touched experts, near
+// what a copy reaches) where the per-token kernels take 255 and 316; a layer of 512 tokens 410 us
+// for 4460.
+template <int NS>
+__global__ __launch_bounds__(GP_BLOCK, NS == 2 ? GP_OCC : 2) void k_native_group_gu(GroupArgs a) {
+    __shared__ __align__(16) gp_abuf3_t abuf;
+    if ((int)blockIdx.y >= *a.n_tiles) return;
+    const GpTile tl = a.tiles[blockIdx.y];
+    const uint8_t *base = a.experts + (size_t)tl.e * a.stride;
+    const uint8_t *const qm[2] = {base + a.off_gq, base + a.off_uq}, *const sm[2] = {base + a.off_gs, base + a.off_us};
+    auto src_row = [&](int i) { return gp_token(a, tl.row + (i < tl.count ? i : 0)); };
+    auto store = [&](int in, int row, const float (&v)[2]) {
+        if (in >= tl.count) return;
+        const int e = a.aexp[src_row(in)];
+        const float g = ldexpf(v[0], e), u = ldexpf(v[1], e);
+        a.out[(size_t)(tl.row + in) * a.F + row] = g / (1.0f + expf(-g)) * u;
+    };
+    gp_with_na<GP_NA_MAX>(__builtin_amdgcn_readfirstlane((tl.count + 15) >> 4),
+                          [&](auto NA) { gn_tile<decltype(NA)::value, 2, NS>(a, a.D, qm, sm, src_row, store, abuf); });
+}
+
+template <int NS>
+__global__ __launch_bounds__(GP_BLOCK, NS == 8 ? 2 : GP_OCC) void k_native_group_down(GroupArgs a) {
+    __shared__ __align__(16) gp_abuf3_t abuf;
+    if ((int)blockIdx.y >= *a.n_tiles) return;
+    const GpTile tl = a.tiles[blockIdx.y];
+    const uint8_t *base = a.experts + (size_t)tl.e * a.stride;
+    const uint8_t *const qm[1] = {base + a.off_dq}, *const sm[1] = {base + a.off_ds};
+    auto src_row = [&](int i) { return tl.row + (i < tl.count ? i : 0); };
+    auto store = [&](int in, int row, const float (&v)[1]) {
+        if (in < tl.count) a.out[(size_t)(tl.row + in) * a.D + row] = ldexpf(v[0], a.aexp[tl.row + in]);
+    };
+    gp_with_na<GP_NA_MAX>(__builtin_amdgcn_readfirstlane((tl.count + 15) >> 4),
+                          [&](auto NA) { gn_tile<decltype(NA)::value, 1, NS>(a, a.F, qm, sm, src_row, store, abuf); });
 }
 
 struct TokenCombineArgs {
