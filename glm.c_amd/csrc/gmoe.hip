@@ -159,11 +159,11 @@ struct gmoe_ctx {
     int *sk_error_host = nullptr;      // pinned host word a failing launch sets (hipHostMalloc)
     // The host-visible outputs (x for the host-buffer forward, xn, shared_out, routed_out,
     // router_prob, topk_w, topk_idx: the pointers above are slices of it, in this order)
-    // in one device block, and its pinned host image: gmoe_forward_host moves a layer's
-    // input and all of its outputs with one copy each way.
+    // in one device block, and a pinned host image that the GPU reads and writes itself:
+    // gmoe_forward_host moves a layer's input and all of its outputs with one kernel each way.
     uint8_t *obs = nullptr, *obs_host = nullptr;
+    float *obs_host_dev = nullptr;  // obs_host's device address
     size_t obs_bytes = 0;
-    float *obs_pack = nullptr;  // a T-token call's parts of obs back to back, and the launch's error word
     int *sk_error_host_dev = nullptr;  // its device address
     unsigned sk_spin_limit = SK_SPIN_LIMIT;
     StackLayer *sk_layers = nullptr;  // [L], device
@@ -237,7 +237,7 @@ static void free_ctx(gmoe_ctx *c) {
         }
         delete[] c->layers;
     }
-    void *bufs[] = {c->obs, c->obs_pack, c->topk_ws, c->h, c->y,
+    void *bufs[] = {c->obs, c->topk_ws, c->h, c->y,
                     c->stage, c->tok_counter, c->panel_counter, c->offsets, c->tokens, c->slots, c->hist_idx, c->hist_w,
                     c->stats_dev, c->staging, c->sk_ws, c->sk_ctr, c->sk_error, c->sk_par_dev,
                     c->sk_layers, c->sk_trace, c->xspl, c->hspl, c->xexp, c->hexp, c->pair_row, c->n_tiles,
@@ -359,9 +359,8 @@ extern "C" int gmoe_create(gmoe_ctx **out, int device, const gmoe_config *cfg) {
         // topk_idx [T][K] -- 4-byte elements, in this order (obs_slice)
         c->obs_bytes = (4 * T * D + T * E + 2 * T * K + 1) * sizeof(float);
         rc |= dev_alloc(&c->obs, c->obs_bytes);
-        rc |= dev_alloc(&c->obs_pack, c->obs_bytes / sizeof(float));
-        if (!rc && hipHostMalloc((void **)&c->obs_host, c->obs_bytes, hipHostMallocDefault) != hipSuccess) {
-            c->obs_host = nullptr;
+        if (!rc && (hipHostMalloc((void **)&c->obs_host, c->obs_bytes, hipHostMallocDefault) != hipSuccess ||
+                    hipHostGetDevicePointer((void **)&c->obs_host_dev, c->obs_host, 0) != hipSuccess)) {
             set_err("hipHostMalloc of %zu bytes failed", c->obs_bytes);
             rc |= GMOE_ERR_NOMEM;
         }
@@ -1344,13 +1343,18 @@ static int copy_out(void *dst, const void *src, size_t bytes) {
     return GMOE_OK;
 }
 
-extern "C" int gmoe_read_layer_state(gmoe_ctx *c, gmoe_layer_state *o, void *stream);
+// n floats (a multiple of 4) of the pinned host image into device memory.
+__global__ __launch_bounds__(256) void k_obs_in(const float4 *__restrict__ host, float4 *__restrict__ x, size_t n4) {
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (size_t)gridDim.x * 256) x[i] = host[i];
+}
 
 // The first T rows of obs's seven arrays (x, xn, shared_out, routed_out [T][D]; router_prob
-// [T][E]; topk_w, topk_idx [T][K]) back to back into pack, then the persistent launch's error
-// word (0 without one): a T-token call's observables leave the device in one copy.
-__global__ __launch_bounds__(256) void k_obs_pack(const float *__restrict__ obs, float *__restrict__ pack, int T, int TM,
-                                                  int D, int E, int K, const int *__restrict__ err) {
+// [T][E]; topk_w, topk_idx [T][K]) back to back into the pinned host image, then the persistent
+// launch's error word (0 without one): a T-token call's observables leave the device in one
+// kernel. (A copy of a packed device buffer instead cost a launch of the runtime's and its own
+// host work: with the input's, 10 to 15 us a call.)
+__global__ __launch_bounds__(256) void k_obs_out(const float *__restrict__ obs, float *__restrict__ pack, int T, int TM,
+                                                 int D, int E, int K, const int *__restrict__ err) {
     const size_t TD = (size_t)T * D, n = 4 * TD + (size_t)T * E + 2 * (size_t)T * K;
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i <= n; i += (size_t)gridDim.x * 256) {
         if (i == n) {
@@ -1359,7 +1363,8 @@ __global__ __launch_bounds__(256) void k_obs_pack(const float *__restrict__ obs,
         }
         size_t src;
         if (i < 4 * TD) {
-            src = (i / TD) * (size_t)TM * D + i % TD;  // array i / TD, row-major [T][D] prefix
+            const int m = (i >= TD) + (i >= 2 * TD) + (i >= 3 * TD);
+            src = i + (size_t)m * (TM - T) * D;  // array m, row-major [T][D] prefix
         } else {
             const size_t j = i - 4 * TD, TE = (size_t)T * E, TK = (size_t)T * K;
             const size_t base = 4 * (size_t)TM * D;
@@ -1368,6 +1373,19 @@ __global__ __launch_bounds__(256) void k_obs_pack(const float *__restrict__ obs,
         }
         pack[i] = obs[src];
     }
+}
+
+// The per-expert lists of T tokens' selections (as k_dispatch forms them: ascending token
+// ids, entries outside the experts skipped): offsets [E + 1] and tokens, either may be null.
+static void host_lists(const int *topk_idx, int T, int K, int E, int32_t *offsets, int32_t *tokens) {
+    int at[GM_MAX_E + 1] = {0};
+    for (int i = 0; i < T * K; i++)
+        if (topk_idx[i] >= 0 && topk_idx[i] < E) at[topk_idx[i] + 1]++;
+    for (int e = 0; e < E; e++) at[e + 1] += at[e];
+    if (offsets) memcpy(offsets, at, (size_t)(E + 1) * sizeof(int));
+    if (!tokens) return;
+    for (int i = 0; i < T * K; i++)
+        if (topk_idx[i] >= 0 && topk_idx[i] < E) tokens[at[topk_idx[i]]++] = i / K;
 }
 
 extern "C" int gmoe_forward_host(gmoe_ctx *c, int layer, int T, const float *x_in, float *x_out, int flags,
@@ -1383,20 +1401,20 @@ extern "C" int gmoe_forward_host(gmoe_ctx *c, int layer, int T, const float *x_i
     HIP_OK(hipSetDevice(c->device));
     const size_t T_ = (size_t)T, TM = (size_t)c->Tmax, D = c->D, E = c->E, K = c->K;
     const size_t bytes = T_ * D * sizeof(float);
-    // in: through the pinned image, one copy
-    float *h = (float *)c->obs_host;
-    memcpy(h, x_in, bytes);
-    HIP_OK(hipMemcpyAsync(c->x_host_io, h, bytes, hipMemcpyHostToDevice, nullptr));
+    // in: through the pinned image
+    memcpy(c->obs_host, x_in, bytes);
+    const size_t n4 = T_ * D / 4;  // D is a multiple of 256
+    hipLaunchKernelGGL(k_obs_in, dim3((unsigned)std::min<size_t>((n4 + 255) / 256, 1024)), dim3(256), 0, nullptr,
+                       (const float4 *)c->obs_host_dev, (float4 *)c->x_host_io, n4);
+    HIP_OK(hipGetLastError());
     int rc = gmoe_forward(c, layer, T, c->x_host_io, c->x_host_io, flags, nullptr);
     if (rc) return rc;
-    // out: x, the observables and the launch's error word packed on the device, one copy, one
-    // synchronisation
+    // out: x, the observables and the launch's error word, one synchronisation
     const size_t TD = T_ * D, n = 4 * TD + T_ * E + 2 * T_ * K;
     const int *err_dev = c->stack_launched && c->stack_last ? c->stack_error_dev : nullptr;
-    hipLaunchKernelGGL(k_obs_pack, dim3((unsigned)std::min<size_t>((n + 256) / 256, 1024)), dim3(256), 0, nullptr,
-                       (const float *)c->obs, c->obs_pack, T, (int)TM, (int)D, (int)E, (int)K, err_dev);
+    hipLaunchKernelGGL(k_obs_out, dim3((unsigned)std::min<size_t>((n + 256) / 256, 1024)), dim3(256), 0, nullptr,
+                       (const float *)c->obs, c->obs_host_dev, T, (int)TM, (int)D, (int)E, (int)K, err_dev);
     HIP_OK(hipGetLastError());
-    HIP_OK(hipMemcpyAsync(c->obs_host, c->obs_pack, (n + 1) * sizeof(float), hipMemcpyDeviceToHost, nullptr));
     HIP_OK(hipStreamSynchronize(nullptr));
     const float *ho = (const float *)c->obs_host;
     // a timed-out launch leaves x_out untouched, so a caller may rerun the layer from it
@@ -1415,15 +1433,10 @@ extern "C" int gmoe_forward_host(gmoe_ctx *c, int layer, int T, const float *x_i
     if (state->routed_out) memcpy(state->routed_out, ho + 3 * TD, bytes);
     if (state->router_prob) memcpy(state->router_prob, ho + 4 * TD, T_ * E * sizeof(float));
     if (state->topk_w) memcpy(state->topk_w, ho + 4 * TD + T_ * E, T_ * K * sizeof(float));
-    if (state->topk_idx) memcpy(state->topk_idx, ho + 4 * TD + T_ * E + T_ * K, T_ * K * sizeof(int));
-    if (state->expert_offsets || state->expert_tokens) {
-        // the per-expert lists (dispatched on demand at T=1) take the general read-back
-        gmoe_layer_state lists;
-        memset(&lists, 0, sizeof(lists));
-        lists.expert_offsets = state->expert_offsets;
-        lists.expert_tokens = state->expert_tokens;
-        return gmoe_read_layer_state(c, &lists, nullptr);
-    }
+    const int *idx = (const int *)(ho + 4 * TD + T_ * E + T_ * K);
+    if (state->topk_idx) memcpy(state->topk_idx, idx, T_ * K * sizeof(int));
+    if (state->expert_offsets || state->expert_tokens)
+        host_lists(idx, T, (int)K, (int)E, state->expert_offsets, state->expert_tokens);
     return GMOE_OK;
 }
 
