@@ -1,12 +1,12 @@
 // gemm.h -- the dense Q8_0 products of a prefill batch (matvec_q80_rows, infer.c:765-786,
 // for every token of the batch) as MFMA GEMMs: each weight panel is read once per tile of
-// up to QG_TT tokens instead of once per token.
+// up to QG_TT_MAX tokens instead of once per token.
 //
 //   k_norm_split  each token's input row, normalised as glm.c normalises it when the
 //                 product takes rmsnorm(x) * w (infer.c:746-752), in the split form of the
 //                 grouped expert GEMMs (grouped.h): fp16 hi and lo with one exponent per row;
 //   k_gemm_q8     y[t][r] = sum_g s[r][g] * (q[r][g] . x_t[g]) for a tile of 64 rows of the
-//                 matrix (four waves of 16) and up to QG_TT tokens, with epilogues for glm.c's
+//                 matrix (four waves of 16) and up to QG_TT_MAX tokens, with epilogues for glm.c's
 //                 SwiGLU pair (infer.c:1078-1080) and residual add (infer.c:1061, 1083).
 //
 // Weights stay in glm.c's row-major Q8_0 form with fp32 scales, which the decode products
@@ -29,8 +29,7 @@
 #include "common.h"
 
 #define QG_BLOCK 256
-#define QG_TT 32                // tokens per tile (two A tiles of 16): twice the blocks of 64-token
-                                // tiles, which leave most CUs idle at a 512-token batch's small matrices
+#define QG_TT_MAX 64            // tokens per tile: 32 or 64 (qg_tokens)
 #define QG_KC 64                // columns per staged chunk
 #define QG_RB (QG_KC * 2)       // bytes of one staged row (one plane of one token)
 #define QG_RG (QG_RB / 16)      // 16-byte groups per staged row
@@ -50,6 +49,8 @@ struct QgArgs {
     int rows, cols, gs, n, xcols, ldy, ldr;
     int x_rows, x_stride;      // row group g (x_rows rows) reads split columns g * x_stride ..
     int bpg, groups, tiles;    // 64-row blocks per group, groups, token tiles
+    float *y_b;                // QG_PLAIN with rows_b > 0: also y_b[t * rows_b + r] = q2 (scales s2) . v,
+    int rows_b;                // rows_b rows of the same columns
 };
 
 typedef _Float16 qg_h8 __attribute__((ext_vector_type(8)));
@@ -163,13 +164,13 @@ __device__ static inline qg_h4 qg_i8_to_h4(unsigned u) {
 // pipeline's exact vmcnt counts. (Weights loaded into registers instead make the compiler
 // wait, at the pipeline loop's join, for every outstanding load, the next chunk's
 // included.)
-//   act  [QG_TT tokens][2 planes][QG_KC] fp16, row r = 2 token + plane, its 16-byte groups
+//   act  [TT tokens][2 planes][QG_KC] fp16, row r = 2 token + plane, its 16-byte groups
 //        XOR-swizzled by token % 8 so that an A-operand read (16 tokens) spreads over the banks;
 //   w    [NM matrices][64 rows][QG_KC] int8, row r's 16-byte groups swizzled by (r / 4) % 4;
 //   s    [NM][256] fp32: row r's scales of the chunk's NB blocks at r NB + b.
-template <int NM>
+template <int NM, int TT>
 struct QgStageBuf {
-    uint8_t act[QG_TT * 2 * QG_RB];
+    uint8_t act[TT * 2 * QG_RB];
     uint8_t w[NM][64 * QG_KC];
     float s[NM][QG_BLOCK];
 };
@@ -191,7 +192,7 @@ struct QgSrc {
 
 template <int NA, int KB, int NM>
 __device__ static inline QgSrc<NA> qg_src_init(const QgArgs &a, int t0, int c_off, int row0, int nrows) {
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x & (QG_BLOCK - 1);
     const int ng = a.cols / KB;
     QgSrc<NA> g;
     g.act0 = a.xs + (size_t)t0 * 2 * a.xcols + c_off;
@@ -217,9 +218,9 @@ __device__ static inline QgSrc<NA> qg_src_init(const QgArgs &a, int t0, int c_of
     return g;
 }
 
-template <int NA, int KB, int NM>
-__device__ static inline void qg_issue(const QgArgs &a, const QgSrc<NA> &g, QgStageBuf<NM> &sb, int c0) {
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+template <int NA, int KB, int NM, int TT>
+__device__ static inline void qg_issue(const QgArgs &a, const QgSrc<NA> &g, QgStageBuf<NM, TT> &sb, int c0) {
+    const int w = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
     const __half *act = g.act0 + c0;
     const int8_t *wq = g.w0 + c0;
     const float *ws = g.s0 + c0 / KB;
@@ -323,17 +324,19 @@ __device__ static inline void qg_mma(const uint8_t *act, const uint8_t *wm, cons
 // and for the wave's shared-memory reads of the chunk before, then on the block, after which
 // that chunk's stage takes the next chunk while this one is multiplied. (Three, four and six
 // stages measured no faster at 201 and 1024 tokens: what a chunk cost was its instructions.)
-template <int NA, int KB, int MODE, int NM>
+template <int NA, int KB, int MODE, int NM, int TT, int NH>
 __device__ __attribute__((always_inline)) static void qg_tile(const QgArgs &a, int panel, int tt,
-                                                             QgStageBuf<NM> (&buf)[2]) {
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+                                                             QgStageBuf<NM, TT> (&bufs)[NH][2]) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int half = NH == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid / QG_BLOCK), w = (tid >> 6) & 3;
+    QgStageBuf<NM, TT>(&buf)[2] = bufs[half];
     const int g = panel / a.bpg, rb = panel % a.bpg;
     const int row0 = g * a.x_rows + 64 * rb;                         // the panel's first row
     const int left = min(a.x_rows - 64 * rb, a.rows - row0);
     const int nrows = left < 64 ? left : 64;                         // its rows (of 64)
     const int pr = 16 * w + (lane & 15);                             // the lane's panel row
     const bool row_on = pr < nrows;
-    const int t0 = QG_TT * tt;
+    const int t0 = TT * tt;
     const QgSrc<NA> src = qg_src_init<NA, KB, NM>(a, t0, g * a.x_stride, row0, nrows);
     float acc[NA][4], acc2[NA][4];
 #pragma unroll
@@ -341,16 +344,42 @@ __device__ __attribute__((always_inline)) static void qg_tile(const QgArgs &a, i
 #pragma unroll
         for (int k = 0; k < 4; k++) acc[i][k] = acc2[i][k] = 0.0f;
     const int nkc = (a.cols + QG_KC - 1) / QG_KC;
-    auto compute = [&](const QgStageBuf<NM> &sb, int kc) {
+    auto compute = [&](const QgStageBuf<NM, TT> &sb, int kc) {
         qg_mma<NA, KB>(sb.act, sb.w[0], sb.s[0], a.cols - kc * QG_KC, pr, acc);
         if (NM == 2) qg_mma<NA, KB>(sb.act, sb.w[NM - 1], sb.s[NM - 1], a.cols - kc * QG_KC, pr, acc2);
     };
-    qg_issue<NA, KB, NM>(a, src, buf[0], 0);
-    for (int kc = 0; kc < nkc; kc++) {
+    // half h's chunks are h, h + NH, ...
+    if (half < nkc) qg_issue<NA, KB, NM, TT>(a, src, buf[0], half * QG_KC);
+    for (int j = 0; j * NH < nkc; j++) {
+        const int kc = j * NH + half;
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();  // chunk kc has landed, and chunk kc - 1 is done with
-        if (kc + 1 < nkc) qg_issue<NA, KB, NM>(a, src, buf[(kc + 1) & 1], (kc + 1) * QG_KC);
-        compute(buf[kc & 1], kc);
+        __builtin_amdgcn_s_barrier();  // chunk kc has landed, and chunk kc - NH is done with
+        if (kc + NH < nkc) qg_issue<NA, KB, NM, TT>(a, src, buf[(j + 1) & 1], (kc + NH) * QG_KC);
+        if (kc < nkc) compute(buf[j & 1], kc);
+    }
+    if (NH == 2) {
+        // the odd chunks' sums through shared memory (the stages, once every wave is done with them)
+        float *x = reinterpret_cast<float *>(&bufs[0][0]) + (tid & (QG_BLOCK - 1));
+        static_assert(NH == 1 || sizeof(bufs) >= sizeof(float) * 8 * NA * QG_BLOCK, "the sums fit the stages");
+        __syncthreads();
+        if (half == 1) {
+#pragma unroll
+            for (int i = 0; i < NA; i++)
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    x[QG_BLOCK * (4 * i + k)] = acc[i][k];
+                    if (NM == 2) x[QG_BLOCK * (4 * (NA + i) + k)] = acc2[i][k];
+                }
+        }
+        __syncthreads();
+        if (half == 1) return;
+#pragma unroll
+        for (int i = 0; i < NA; i++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                acc[i][k] = __fadd_rn(acc[i][k], x[QG_BLOCK * (4 * i + k)]);
+                if (NM == 2) acc2[i][k] = __fadd_rn(acc2[i][k], x[QG_BLOCK * (4 * (NA + i) + k)]);
+            }
     }
     // lane l holds tokens 16 i + 4 (l / 16) + k of panel row pr
     const int r = row0 + pr;
@@ -398,18 +427,44 @@ __device__ __attribute__((always_inline)) static inline void qg_with_na(int na, 
 // wave, and everything else in it has to stay near that. Hence scalar base addresses stepped
 // along the rows (no vector instruction a DMA, no division by the group size), operands read
 // together, the accumulators in vector registers (launch bounds that leave the matrix cores no
-// use for their own, whose every read is an instruction). Before and after, us: group size 16,
-// 201 tokens: attn_out 74 -> 52, layer 0's gate/up 137 -> 84, q_a 30 -> 22; group size 32, 1024
-// tokens: attn_out 107 -> 98, gate/up 318 -> 275.
-template <int KB, int MODE>
-__global__ __launch_bounds__(QG_BLOCK, MODE == QG_PAIR ? 3 : 4) void k_gemm_q8(QgArgs a) {
+// use for their own, whose every read is an instruction). Before and after, us, with the rules
+// below: group size 16, 201 tokens: attn_out 74 -> 41, layer 0's gate/up 137 -> 84, q_a and kv_a
+// 30 + 30 -> 18; group size 32, 1024 tokens: attn_out 107 -> 79, gate/up 318 -> 240.
+template <int KB, int MODE, int TT, int NH>
+__global__ __launch_bounds__(QG_BLOCK *NH, NH == 2 ? 2 : TT > 32 ? (MODE == QG_PAIR || KB == 16 ? 2 : 3) : MODE == QG_PAIR ? 3 : 4)
+void k_gemm_q8(QgArgs a) {
     constexpr int NM = MODE == QG_PAIR ? 2 : 1;
-    __shared__ __align__(16) QgStageBuf<NM> buf[2];
+    __shared__ __align__(16) QgStageBuf<NM, TT> buf[NH][2];
     const int b = blockIdx.x, xcd = b % QG_XCD, k = b / QG_XCD;
-    const int ppx = (a.bpg * a.groups + QG_XCD - 1) / QG_XCD;  // panels per XCD
-    const int panel = (k % ppx) * QG_XCD + xcd, tt = k / ppx;
-    if (panel >= a.bpg * a.groups) return;
-    const int left = a.n - QG_TT * tt;
-    const int na = __builtin_amdgcn_readfirstlane(left >= QG_TT ? QG_TT / 16 : (left + 15) >> 4);
-    qg_with_na<QG_TT / 16>(na, [&](auto NA) { qg_tile<decltype(NA)::value, KB, MODE, NM>(a, panel, tt, buf); });
+    const int na_ = a.bpg * a.groups, nb_ = a.rows_b ? (a.rows_b + 63) / 64 : 0;  // panels of the matrix, of the second
+    const int ppx = (na_ + nb_ + QG_XCD - 1) / QG_XCD;  // panels per XCD
+    int panel = (k % ppx) * QG_XCD + xcd;
+    const int tt = k / ppx;
+    if (panel >= na_ + nb_) return;
+    if (MODE == QG_PLAIN && panel >= na_) {  // the second product of the same inputs
+        panel -= na_;
+        a.q = a.q2;
+        a.s = a.s2;
+        a.y = a.y_b;
+        a.rows = a.x_rows = a.rows_b;
+        a.bpg = nb_;
+        a.ldy = a.rows_b;
+    }
+    const int left = a.n - TT * tt;
+    const int na = __builtin_amdgcn_readfirstlane(left >= TT ? TT / 16 : (left + 15) >> 4);
+    qg_with_na<TT / 16>(na, [&](auto NA) { qg_tile<decltype(NA)::value, KB, MODE, NM, TT, NH>(a, panel, tt, buf); });
 }
+
+// Tokens per tile for n tokens and `panels` 64-row panels on n_cu compute units: 64 where that
+// leaves every CU two blocks (a chunk's weights are converted once for twice the tokens) and the
+// rows are long enough for it to tell, else 32, which is twice the blocks. 1024 tokens at group
+// size 32, 32 and 64 tokens a tile: attn_out (5120 columns) 98 and 79 us, layer 0's gate/up (2048)
+// 275 and 240, q_b (768) 34.3 and 34.0, k_b (192) 30.2 and 34.2.
+static inline int qg_tokens(int n, int panels, int cols, int n_cu) {
+    return cols >= 1024 && (size_t)panels * ((n + 63) / 64) >= 2 * (size_t)n_cu ? 64 : 32;
+}
+// Whether the 32-token tiles' blocks run two halves of four waves, each every other chunk: where
+// there are too few blocks to give each SIMD two waves of them, which hide each other's waits. 201
+// tokens at group size 16: attn_out (224 blocks) 52 and 41 us; q_a and kv_a (147 blocks in one
+// launch) 18 us, where a launch each took 22.
+static inline bool qg_halves(int n, int panels, int n_cu) { return (size_t)panels * ((n + 31) / 32) < 2 * (size_t)n_cu; }

@@ -461,7 +461,7 @@ int dense_ffn(gmoe_model *m, hipStream_t st) {
 // (token t reads positions up to pos0 + t only), then the attention over the cache runs
 // per token, since its length differs.
 // Whether a batch of n tokens takes the GEMMs of gemm.h for its dense products (a weight
-// panel read once per QG_TT tokens) rather than k_gemv per token: a batch of a few tokens
+// panel read once per tile of 32 or 64 tokens) rather than k_gemv per token: a batch of a few tokens
 // gains nothing from tiles. Group sizes 16 (glm.c's exporter) and 32 take it.
 bool gemm_batch(const gmoe_model *m, int n) {
     const int gs = m->c.group_size;
@@ -478,13 +478,32 @@ void gemm_inputs(gmoe_model *m, const float *x, int ldx, int cols, const float *
     else hipLaunchKernelGGL(k_norm_split<QG_SPLIT_MAX>, grid, block, 0, st, x, ldx, cols, norm, m->xs, m->xe);
 }
 
+// k_gemm_q8's launch with TT tokens a tile and NH halves a block.
+template <int TT, int NH>
+void gemm_tiles(QgArgs a, int mode, int panels, hipStream_t st) {
+    a.tiles = (a.n + TT - 1) / TT;
+    const dim3 grid((unsigned)(QG_XCD * ((panels + QG_XCD - 1) / QG_XCD) * a.tiles)), block(QG_BLOCK * NH);
+    if (a.gs == 32) {  // gemm_batch: 16 or 32, the kernel's block of columns with one scale
+        if (mode == QG_PAIR) hipLaunchKernelGGL((k_gemm_q8<32, QG_PAIR, TT, NH>), grid, block, 0, st, a);
+        else if (mode == QG_RESID) hipLaunchKernelGGL((k_gemm_q8<32, QG_RESID, TT, NH>), grid, block, 0, st, a);
+        else hipLaunchKernelGGL((k_gemm_q8<32, QG_PLAIN, TT, NH>), grid, block, 0, st, a);
+    } else {
+        if (mode == QG_PAIR) hipLaunchKernelGGL((k_gemm_q8<16, QG_PAIR, TT, NH>), grid, block, 0, st, a);
+        else if (mode == QG_RESID) hipLaunchKernelGGL((k_gemm_q8<16, QG_RESID, TT, NH>), grid, block, 0, st, a);
+        else hipLaunchKernelGGL((k_gemm_q8<16, QG_PLAIN, TT, NH>), grid, block, 0, st, a);
+    }
+}
+
 // y = q . v for the n tokens' split inputs (gemm_inputs, cols columns): rows of group g
 // (x_rows each) read input columns g * x_stride .. (x_rows = rows: one group); mode
-// QG_PLAIN, QG_RESID (y = resid + dot) or QG_PAIR (y = silu(q . v) * (q2 . v)).
+// QG_PLAIN, QG_RESID (y = resid + dot) or QG_PAIR (y = silu(q . v) * (q2 . v)); with rows_b
+// (QG_PLAIN, one group) also y_b = q2 . v, rows_b rows, in the same launch.
 void gemm_launch(gmoe_model *m, const int8_t *q, const float *s, const int8_t *q2, const float *s2, int rows, int cols,
                  int x_rows, int x_stride, int xcols, float *y, int ldy, const float *resid, int ldr, int mode, int n,
-                 hipStream_t st) {
+                 hipStream_t st, float *y_b = nullptr, int rows_b = 0) {
     QgArgs a{};
+    a.y_b = y_b;
+    a.rows_b = rows_b;
     a.q = q;
     a.s = s;
     a.q2 = q2;
@@ -505,18 +524,10 @@ void gemm_launch(gmoe_model *m, const int8_t *q, const float *s, const int8_t *q
     a.x_stride = x_stride;
     a.bpg = (x_rows + 63) / 64;
     a.groups = (rows + x_rows - 1) / x_rows;
-    a.tiles = (n + QG_TT - 1) / QG_TT;
-    const int panels = a.bpg * a.groups;
-    const dim3 grid((unsigned)(QG_XCD * ((panels + QG_XCD - 1) / QG_XCD) * a.tiles));
-    if (a.gs == 32) {  // gemm_batch: 16 or 32, the kernel's block of columns with one scale
-        if (mode == QG_PAIR) hipLaunchKernelGGL((k_gemm_q8<32, QG_PAIR>), grid, dim3(QG_BLOCK), 0, st, a);
-        else if (mode == QG_RESID) hipLaunchKernelGGL((k_gemm_q8<32, QG_RESID>), grid, dim3(QG_BLOCK), 0, st, a);
-        else hipLaunchKernelGGL((k_gemm_q8<32, QG_PLAIN>), grid, dim3(QG_BLOCK), 0, st, a);
-    } else {
-        if (mode == QG_PAIR) hipLaunchKernelGGL((k_gemm_q8<16, QG_PAIR>), grid, dim3(QG_BLOCK), 0, st, a);
-        else if (mode == QG_RESID) hipLaunchKernelGGL((k_gemm_q8<16, QG_RESID>), grid, dim3(QG_BLOCK), 0, st, a);
-        else hipLaunchKernelGGL((k_gemm_q8<16, QG_PLAIN>), grid, dim3(QG_BLOCK), 0, st, a);
-    }
+    const int panels = a.bpg * a.groups + (rows_b + 63) / 64;
+    if (qg_tokens(n, panels, cols, m->n_cu) == 64) gemm_tiles<64, 1>(a, mode, panels, st);
+    else if (qg_halves(n, panels, m->n_cu)) gemm_tiles<32, 2>(a, mode, panels, st);
+    else gemm_tiles<32, 1>(a, mode, panels, st);
 }
 
 int attention_batch(gmoe_model *m, int l, int pos0, int n, hipStream_t st) {
@@ -526,9 +537,9 @@ int attention_batch(gmoe_model *m, int l, int pos0, int n, hipStream_t st) {
     const int ql = c.q_lora_rank, hk = c.head_k_dim, vh = c.v_head_dim;
     if (gemm_batch(m, n)) {
         gemm_inputs(m, m->x, D, D, A.attn_norm, n, st);
-        gemm_launch(m, A.q_a_q, A.q_a_s, nullptr, nullptr, ql, D, ql, 0, D, m->q_a, ql, nullptr, 0, QG_PLAIN, n, st);
-        gemm_launch(m, A.kv_a_q, A.kv_a_s, nullptr, nullptr, kv + rope, D, kv + rope, 0, D, m->kv_a, kv + rope, nullptr,
-                    0, QG_PLAIN, n, st);
+        // q_a and kv_a, two small products of the same inputs, in one launch
+        gemm_launch(m, A.q_a_q, A.q_a_s, A.kv_a_q, A.kv_a_s, ql, D, ql, 0, D, m->q_a, ql, nullptr, 0, QG_PLAIN, n, st,
+                    m->kv_a, kv + rope);
         gemm_inputs(m, m->q_a, ql, ql, A.q_a_norm, n, st);
         gemm_launch(m, A.q_b_q, A.q_b_s, nullptr, nullptr, H * hk, ql, H * hk, 0, ql, m->q_full, H * hk, nullptr, 0,
                     QG_PLAIN, n, st);
