@@ -2,8 +2,9 @@
 // is a multiple of 16 and fp32 scales as the exporter writes them (scale = max|w| / 127,
 // which fp16 cannot hold in general). The matrices stay in the checkpoint layout, int8
 // [rows][cols] with fp32 scales [rows][cols/gs] (infer.c:707-739); a context in this form
-// runs these kernels for every T (the tiled decode and prefill kernels assume gs = 32 and
-// fp16-exact scales).
+// runs these kernels at T = 1 and for small batches, which read an expert once per (token,
+// slot), and k_native_group_gu and k_native_group_down (grouped.h) for larger ones (the tiled
+// decode and prefill kernels assume gs = 32 and fp16-exact scales).
 //
 // A matrix row's dot product is one wave's: the row is cut into 16-column units, lane l
 // takes units l and l + 64 (cols <= 2048), and a unit lies inside one group, so each unit's

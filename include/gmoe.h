@@ -65,8 +65,9 @@ typedef struct gmoe_config {
  *   decode kernels and the grouped prefill GEMMs run on this form.
  * NATIVE: glm.c's own layout, int8 rows and fp32 scales, for any group size that is a
  *   multiple of 16 and divides dim and moe_ffn_dim (the exporter writes group size 16 and
- *   scales max|w|/127, glm47_flash_export.py:36,157-169). Every T runs the native
- *   kernels: one wave per matrix row, each group's sum scaled by its own fp32 scale.
+ *   scales max|w|/127, glm47_flash_export.py:36,157-169). T=1 and small batches run one
+ *   wave per matrix row, each group's sum scaled by its own fp32 scale; larger batches (from
+ *   T (K + 1) = E + 2 K) grouped GEMMs over the same rows.
  * TILED16: the exporter's form on the fast path: group size 16, fp32 scales kept exactly
  *   as they are, q planes tiled as in TILED. T=1 runs the persistent relay decode kernel
  *   (k_moe_relay), T>1 the grouped prefill GEMMs; gmoe_create refuses it where the shape
