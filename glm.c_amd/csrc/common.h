@@ -43,6 +43,9 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 
 typedef __attribute__((address_space(3))) void lds_void;
 
+// An LDS DMA's destination into m0, with the wait state that a scalar write of m0 needs before
+// the DMA reads it: inside an asm statement the compiler's hazard pass does not put it there.
+#define GM_M0(op) "s_mov_b32 m0, " op "\n\ts_nop 0\n\t"
 // One 16-byte piece per lane from global memory straight into shared memory (lane l at
 // dst + 16 l), issued by inline assembly, which the compiler does not see as a
 // shared-memory DMA: with a global_load_lds of its own in flight, the compiler waits for
@@ -51,7 +54,7 @@ typedef __attribute__((address_space(3))) void lds_void;
 // `dst`.
 __device__ static inline void dma16_untracked(const GM_GLOBAL void *src, lds_void *dst) {
     const unsigned m0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)dst);
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(m0) : "memory", "m0");
+    asm volatile(GM_M0("%1") "global_load_lds_dwordx4 %0, off" ::"v"(src), "s"(m0) : "memory", "m0");
 }
 // The same, BYTES (4 or 16) per lane, from the scalar address base plus the lane's byte offset,
 // so that stepping base along a row costs no vector instruction.
@@ -59,9 +62,9 @@ template <int BYTES>
 __device__ static inline void dma_s(const void *base, unsigned off, const lds_void *dst) {
     const unsigned m0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)dst);
     if (BYTES == 16)
-        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
+        asm volatile(GM_M0("%2") "global_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
     else
-        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
+        asm volatile(GM_M0("%2") "global_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
 }
 // N (at most 4) consecutive pieces of 1 KB, 16 bytes per lane each: piece i from base + 1024 i
 // to dst + 1024 i, by the instruction's offset, which applies to both.
@@ -70,14 +73,14 @@ __device__ static inline void dma_run(const void *base, unsigned off, const lds_
     const unsigned m0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)dst);
 #define GM_DMA "global_load_lds_dwordx4 %0, %1"
     if (N == 1)
-        asm volatile("s_mov_b32 m0, %2\n\t" GM_DMA ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
+        asm volatile(GM_M0("%2") GM_DMA ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
     else if (N == 2)
-        asm volatile("s_mov_b32 m0, %2\n\t" GM_DMA "\n\t" GM_DMA " offset:1024" ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
+        asm volatile(GM_M0("%2") GM_DMA "\n\t" GM_DMA " offset:1024" ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
     else if (N == 3)
-        asm volatile("s_mov_b32 m0, %2\n\t" GM_DMA "\n\t" GM_DMA " offset:1024\n\t" GM_DMA " offset:2048" ::"v"(off), "s"(base),
+        asm volatile(GM_M0("%2") GM_DMA "\n\t" GM_DMA " offset:1024\n\t" GM_DMA " offset:2048" ::"v"(off), "s"(base),
                      "s"(m0) : "memory", "m0");
     else
-        asm volatile("s_mov_b32 m0, %2\n\t" GM_DMA "\n\t" GM_DMA " offset:1024\n\t" GM_DMA " offset:2048\n\t" GM_DMA
+        asm volatile(GM_M0("%2") GM_DMA "\n\t" GM_DMA " offset:1024\n\t" GM_DMA " offset:2048\n\t" GM_DMA
                      " offset:3072" ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
 #undef GM_DMA
 }

@@ -1,0 +1,80 @@
+"""The built GPU code held to rules of the instruction set that inline assembly can break
+without an error: what the compiler's hazard pass sees to by itself for its own instructions, it
+cannot see inside an asm statement."""
+import os
+import re
+import struct
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIB = os.path.join(ROOT, "glm.c_amd", "libgmoe.so")
+OBJDUMP = os.path.join(os.environ.get("ROCM", "/opt/rocm"), "llvm", "bin", "llvm-objdump")
+MAGIC = b"__CLANG_OFFLOAD_BUNDLE__"
+
+
+def code_objects():
+    """The gfx950 code objects of libgmoe.so (one per source file), from its offload bundles."""
+    data = open(LIB, "rb").read()
+    found, at = [], data.find(MAGIC)
+    while at >= 0:
+        (n,) = struct.unpack_from("<Q", data, at + len(MAGIC))
+        p = at + len(MAGIC) + 8
+        if n < 16:  # (the magic's own text elsewhere is not a bundle)
+            for _ in range(n):
+                off, size, idlen = struct.unpack_from("<QQQ", data, p)
+                name = data[p + 24:p + 24 + idlen]
+                p += 24 + idlen
+                if b"gfx950" in name and size:
+                    found.append(data[at + off:at + off + size])
+        at = data.find(MAGIC, at + 1)
+    return found
+
+
+@pytest.fixture(scope="module")
+def listing(tmp_path_factory):
+    """[instruction lines] of every code object."""
+    objs = code_objects()
+    assert objs, "no gfx950 code in libgmoe.so"
+    lines = []
+    for i, blob in enumerate(objs):
+        path = tmp_path_factory.mktemp("co") / f"{i}.co"
+        path.write_bytes(blob)
+        out = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", "--no-leading-addr", str(path)], check=True,
+                             capture_output=True, text=True).stdout
+        lines += [re.sub(r"\s*//.*", "", s).strip() for s in out.splitlines() if s.startswith((" ", "\t"))]
+    return lines
+
+
+def test_m0_write_has_a_wait_state_before_a_dma_reads_it(listing):
+    """An LDS DMA takes its destination from m0, and a scalar write of m0 needs one wait state (any
+    other instruction) before it; the compiler puts an s_nop there where it has nothing else."""
+    dma = [i for i, s in enumerate(listing) if re.match(r"(global|buffer)_load_(lds_|.*\blds$)", s)]
+    assert len(dma) > 100, "the listing's DMAs were not recognised"
+    bad = [f"{listing[i - 1]} / {listing[i]}" for i in dma if re.match(r"s_\w+ m0,", listing[i - 1])]
+    assert not bad, f"{len(bad)} of {len(dma)} DMAs read m0 right after its write, e.g. {bad[0]}"
+
+
+def sgprs(text):
+    """The scalar registers that an operand list names."""
+    regs = {int(m) for m in re.findall(r"\bs(\d+)\b", text)}
+    for a, b in re.findall(r"\bs\[(\d+):(\d+)\]", text):
+        regs |= set(range(int(a), int(b) + 1))
+    return regs
+
+
+def test_no_vector_write_of_a_scalar_address_right_before_its_load(listing):
+    """A scalar register that a vector instruction wrote (v_readfirstlane) needs five wait states
+    before a memory instruction takes it as its address."""
+    bad = []
+    for i, s in enumerate(listing):
+        used = sgprs(s) if re.match(r"(global|buffer)_", s) else ()
+        states, j = 0, i - 1
+        while used and states < 5 and j >= 0:
+            op, _, rest = listing[j].partition(" ")
+            if op.startswith("v_") and sgprs(rest.split(",")[0]) & used:
+                bad.append(f"{listing[j]} / {s}")
+            states += int(rest) + 1 if op == "s_nop" else 1
+            j -= 1
+    assert not bad, f"{len(bad)} loads, e.g. {bad[0]}"
