@@ -181,9 +181,8 @@ __global__ __launch_bounds__(A16_BLOCK, 1) void k_attn_tile16(AttnTileArgs g) {
     // on to tile j: this wave's part of it has landed, then every wave's has and none still
     // reads tile j - 1, whose stage takes tile j + 1
     auto next = [&]() {
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        block_barrier();
         if (j + 1 < ntile) issue(r0 + A16_P * (j + 1), (j + 1) & 1);
     };
     a16_h4 vb[3][2][4];  // the weighted sum's operands: see vload

@@ -84,6 +84,12 @@ __device__ static inline void dma_run(const void *base, unsigned off, const lds_
                      " offset:3072" ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
 #undef GM_DMA
 }
+// The block's barrier once the wave's shared-memory reads and writes are done, without
+// __syncthreads()'s wait for the loads and DMAs in flight (the caller waits for what it needs
+// first). In one statement with the wait, so that the compiler moves no memory access over it:
+// __builtin_amdgcn_s_barrier() orders none, and left reads of a buffer still under way at the
+// barrier after which other waves refill it.
+__device__ static inline void block_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 __host__ __device__ static inline size_t gm_q_offset(int r, int c, int cols) {

@@ -401,10 +401,6 @@ __device__ static inline float row_reduce_scatter8(const float (&v)[8], int s) {
     return y + dpp_f<DPP_QUAD_1032>(y);
 }
 
-// A block barrier after this wave's shared-memory accesses only: global loads still in
-// flight (the next tile's) are not waited for, as __syncthreads()'s release fence would.
-__device__ static inline void at_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 #define AT_HB 2  // heads per thread in k_attn_chunk's scores and weighted sum
 #define AT_TB 4  // cache positions per thread in its scores
 static_assert(AT_HB * AT_TB == 8, "row_reduce_scatter8 takes eight scores per lane");
@@ -518,7 +514,7 @@ __global__ __launch_bounds__(AT_BLOCK) void k_attn_chunk(AttnArgs a) {
             ks[tid * ksd + KQ] = 0.0f;
             ks[tid * ksd + KQ + 1] = 0.0f;
         }
-        at_barrier();
+        block_barrier();
         if (t0 + AT_TILE < r1) fetch(t0 + AT_TILE);  // in flight while this tile is used
         // scores: row sg takes heads AT_HB gh .. and positions AT_TB gt .. (rows past nh or nt
         // read LDS rows inside the buffers and are not written)
@@ -550,7 +546,7 @@ __global__ __launch_bounds__(AT_BLOCK) void k_attn_chunk(AttnArgs a) {
             const int h = AT_HB * gh + (sl >> 3), t = AT_TB * gt + ((sl >> 1) & 3);
             if ((sl & 1) == 0 && h < nh && t < nt) sc[h][t] = __fmul_rn(v, a.kq_scale);
         }
-        at_barrier();
+        block_barrier();
         // per head (a wave each): the tile's maximum, the running maximum and sum of
         // exponentials, exp(score - running maximum) for the tile (lane = position; zeros
         // past nt, which the weighted sum reads in its last step)
@@ -567,7 +563,7 @@ __global__ __launch_bounds__(AT_BLOCK) void k_attn_chunk(AttnArgs a) {
                 corr[h] = cr;
             }
         }
-        at_barrier();
+        block_barrier();
         if (summer) {
 #pragma unroll
             for (int x = 0; x < AT_HB; x++) {  // head groups past nh rescale rows that are not stored
@@ -597,7 +593,7 @@ __global__ __launch_bounds__(AT_BLOCK) void k_attn_chunk(AttnArgs a) {
                 }
             }
         }
-        at_barrier();  // the next tile overwrites ks and sc
+        block_barrier();  // the next tile overwrites ks and sc
     }
     if (summer) {
 #pragma unroll

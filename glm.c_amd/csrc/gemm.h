@@ -352,8 +352,8 @@ __device__ __attribute__((always_inline)) static void qg_tile(const QgArgs &a, i
     if (half < nkc) qg_issue<NA, KB, NM, TT>(a, src, buf[0], half * QG_KC);
     for (int j = 0; j * NH < nkc; j++) {
         const int kc = j * NH + half;
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();  // chunk kc has landed, and chunk kc - NH is done with
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        block_barrier();  // chunk kc has landed, and chunk kc - NH is done with
         if (kc + NH < nkc) qg_issue<NA, KB, NM, TT>(a, src, buf[(j + 1) & 1], (kc + NH) * QG_KC);
         if (kc < nkc) compute(buf[j & 1], kc);
     }

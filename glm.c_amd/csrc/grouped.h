@@ -190,10 +190,9 @@ __device__ __attribute__((always_inline)) static inline void gp_with_na(int na, 
 // unrolled by two), k_group_gu two (three sets and buffers, unrolled by three; its
 // gate and up weights make it the larger stream: 162 -> 151 us at T=512, while a third set
 // in k_group_down, at 159 VGPRs and three blocks per CU, was slower), so that the register
-// sets rotate without copies. Barriers are plain s_barrier after an exact vmcnt wait:
+// sets rotate without copies. Barriers are block_barrier() after an exact vmcnt wait:
 // __syncthreads() carries a release fence that waits for every outstanding load, the
 // prefetch included, which would serialise the pipeline.
-__device__ static inline void gp_barrier() { __builtin_amdgcn_s_barrier(); }
 
 typedef uint8_t gp_abuf_t[2][GP_TOK * 2 * GP_RB];
 typedef uint8_t gp_abuf3_t[3][GP_TOK * 2 * GP_RB];  // k_group_gu: two chunks in flight
@@ -305,9 +304,9 @@ __device__ __attribute__((always_inline)) static inline void gp_gu_tile(const Gr
         } else {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
-        gp_barrier();  // every wave's part of chunk kc's activations is in shared memory
+        block_barrier();  // every wave's part of chunk kc's activations is in shared memory
         compute(r, kc);
-        gp_barrier();  // every wave is done with buffer kc % 3 before it is refilled
+        block_barrier();  // every wave is done with buffer kc % 3 before it is refilled
     };
     GuRegs<G16> r0, r1, r2;
     issue(r0, 0);
@@ -406,13 +405,13 @@ __device__ __attribute__((always_inline)) static inline void gp_down_tile(const 
     auto step = [&](DnRegs<G16> &r, DnRegs<G16> &rn, int kc) {
         issue(rn, kc + 1);
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(gp_dn_loads(NA, G16)) : "memory");
-        gp_barrier();
+        block_barrier();
         compute(r, kc);
-        gp_barrier();
+        block_barrier();
     };
     auto last = [&](DnRegs<G16> &r, int kc) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        gp_barrier();
+        block_barrier();
         compute(r, kc);
     };
     DnRegs<G16> r0, r1;
@@ -583,10 +582,9 @@ __device__ __attribute__((always_inline)) static inline void gn_tile(const Group
         } else {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
-        gp_barrier();
+        block_barrier();
         compute(r, kc);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        gp_barrier();
+        block_barrier();
     };
     static_assert(2 * gn_loads(GP_NA_MAX, 2, 8) < 64, "vmcnt counts six bits");
     float first[NM][NA][4];  // the first half of the chunks

@@ -78,3 +78,21 @@ def test_no_vector_write_of_a_scalar_address_right_before_its_load(listing):
             states += int(rest) + 1 if op == "s_nop" else 1
             j -= 1
     assert not bad, f"{len(bad)} loads, e.g. {bad[0]}"
+
+
+def test_no_shared_memory_read_is_under_way_at_a_barrier(listing):
+    """After a barrier other waves (and their DMAs) write what a wave read before it, so its reads
+    have returned by then; __builtin_amdgcn_s_barrier() neither waits for them nor keeps the
+    compiler from moving them over it."""
+    pending, bad = 0, 0
+    for s in listing:
+        wait = re.search(r"lgkmcnt\((\d+)\)", s)
+        if s == "s_endpgm":
+            pending = 0
+        elif wait:
+            pending = min(pending, int(wait[1]))
+        elif s.startswith("ds_read"):
+            pending += 1
+        elif s.startswith("s_barrier"):
+            bad += pending > 0
+    assert bad == 0, f"{bad} barriers with reads of shared memory under way"
