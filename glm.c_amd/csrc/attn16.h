@@ -28,6 +28,8 @@
 // 2^(A16_PUP + e[p] - eR), eR at least every e[p] of the tile, so that fp16 holds them (e^6 2^6 <
 // 2^15); eR follows the tile's largest e upward at once and downward when it is more than
 // A16_EDOWN above it, so that a split exponential's error stays at 2^-25 of the largest's or less.
+// Downward the sum grows by as much, so a step down stops where the sum would pass 2^A16_XMAX, and
+// a tile of zero entries alone, whose products are zero at any scale, moves nothing (a16_scale).
 #pragma once
 
 #include "attn.h"
@@ -40,6 +42,8 @@
 #define A16_SLACK 6.0f
 #define A16_PUP 6
 #define A16_EDOWN 6
+#define A16_EMIN (-200)             // below any entry's exponent (spl_exp: -163 at least)
+#define A16_XMAX 100
 static_assert(AQ_T == 16 * A16_BLOCK / 64, "16 tokens a wave");
 static_assert(AQ_KQ_MAX == SPL_KCOLS && AT_KV_MAX <= SPL_KCOLS, "the split rows hold the widest entry");
 static_assert(A16_STAGE % 16 == 0, "16-byte DMA slots");
@@ -47,6 +51,27 @@ static_assert(16 * SPL_KROW * 2 + 2 * SPL_KCOLS + 2 * AT_KV_MAX < 65536, "one ba
 
 // s_waitcnt immediate (gfx9 encoding) for lgkmcnt(n) alone, n <= 15
 #define A16_WAIT_LGKM(n) (0xC07F | ((n) << 8))
+
+// The scale exponent that follows eR at a tile whose largest is em (SPL_EMPTY: zero entries
+// alone), with the sum's magnitudes below 2^xa (A16_ZERO: the sum is zero, and moves at no cost).
+#define A16_ZERO (-1000)
+__host__ __device__ constexpr int a16_scale(int eR, int em, int xa) {
+    if (em == SPL_EMPTY) return eR;
+    if (em >= eR || xa == A16_ZERO) return em;
+    const int room = xa < A16_XMAX ? A16_XMAX - xa : 0;
+    return em > eR - room ? em : eR - room;
+}
+constexpr bool a16_scale_bounded() {
+    for (int eR = A16_EMIN; eR <= 113; eR += 7)
+        for (int em = -163; em <= 113; em += 12)
+            for (int xa = -126; xa <= 129; xa += 5) {
+                const int e = a16_scale(eR, em, xa), x = xa + eR - e;
+                if (e < em || (e < eR && x > A16_XMAX) || (e > em && e != eR && x != A16_XMAX)) return false;
+                if (a16_scale(eR, SPL_EMPTY, xa) != eR || a16_scale(eR, em, A16_ZERO) != em) return false;
+            }
+    return true;
+}
+static_assert(a16_scale_bounded(), "a step down lands on the tile's exponent or on the sum's bound");
 
 typedef _Float16 a16_h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 a16_h4 __attribute__((ext_vector_type(4)));
@@ -173,7 +198,7 @@ __global__ __launch_bounds__(A16_BLOCK, 1) void k_attn_tile16(AttnTileArgs g) {
 #pragma unroll
     for (int i = 0; i < A16_NCB; i++) acc[i] = (aq_f4){0.0f, 0.0f, 0.0f, 0.0f};
     float m = -INFINITY, l = 0.0f;  // the token's reference score; the lane's part of its sum
-    int eR = 0;                     // the scale of acc: 2^(eR - A16_PUP)
+    int eR = A16_EMIN;              // the scale of acc: 2^(eR - A16_PUP)
 
     // the wave's tiles: those that any of its tokens attends (the later ones it only passes on)
     const int past = a.pos + tw + 15 - r0, nt = past < 0 ? 0 : min(ntile, past / A16_P + 1);
@@ -286,11 +311,21 @@ __global__ __launch_bounds__(A16_BLOCK, 1) void k_attn_tile16(AttnTileArgs g) {
         while (more) {
             {
                 const float mn = fmaxf(m, a16_max4(mx));
-                int eT = __builtin_amdgcn_readfirstlane((int)a16_max4((float)em));  // the same for every l16
-                eT = j == 0 ? max(eT, -200) : max(eT, eR - 60);  // (a zero tile's SPL_EMPTY in bounded steps)
+                const int et = __builtin_amdgcn_readfirstlane((int)a16_max4((float)em));  // the same for every l16
+                int xa = A16_ZERO;
+                if (j > 0 && et < eR) {
+                    float ax = 0.0f;
+#pragma unroll
+                    for (int i = 0; i < A16_NCB; i++)
+#pragma unroll
+                        for (int r = 0; r < 4; r++) ax = fmaxf(ax, fabsf(acc[i][r]));
+                    const unsigned b = __builtin_amdgcn_readfirstlane(__float_as_uint(wave_max_f(ax)));
+                    if (b) xa = (int)(b >> 23) - 126;
+                }
+                const int eT = a16_scale(eR, et, xa);
                 float cr = mn == -INFINITY ? 1.0f : expf(__fsub_rn(m, mn));  // 0 while m is -inf
                 l = __fmul_rn(l, cr);
-                cr = ldexpf(cr, j == 0 ? 0 : eR - eT);
+                cr = ldexpf(cr, eR - eT);
 #pragma unroll
                 for (int i = 0; i < A16_NCB; i++)
 #pragma unroll
@@ -329,7 +364,7 @@ __global__ __launch_bounds__(A16_BLOCK, 1) void k_attn_tile16(AttnTileArgs g) {
                 next();
                 scores();
                 // a score past the reference's slack, or an exponent outside eR's range
-                if (__any(mx > m + A16_SLACK || em > eR) || !__any(em >= eR - A16_EDOWN)) break;
+                if (__any(mx > m + A16_SLACK || em > eR) || (!__any(em >= eR - A16_EDOWN) && __any(em > SPL_EMPTY))) break;
                 exps();
             }
         }

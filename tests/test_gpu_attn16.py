@@ -88,3 +88,61 @@ def test_split_fp16_attention_matches_fp32(name):
         check("8 tokens at 503 after kept and decoded tokens", rng.integers(0, cfg["vocab_size"], 8).astype(np.int32), 503)
     finally:
         model.close()
+
+
+# The running scale and the reference score of a chunk (a16_scale; A16_SLACK): 1024 tokens of 20
+# heads, whose chunks are eleven 32-position tiles. Token 0's embedding row is zero (layer 0's
+# entry of it is exactly zero), those of tokens 1..3 are scaled by 2^-36, 2^-56 and 2^-76 (their
+# entries, which come from x / sqrt(mean x^2 + 1e-5), lie about 2^-21, 2^-41 and 2^-61 of an ordinary
+# token's); "scores" multiplies the queries by 4, which leaves the scores a standard deviation of
+# 4 and 14, so that a chunk's maximum passes the slack several times.
+def tall(**over):
+    cfg = dict(small(), n_heads=20, cache_cap=1152, max_batch=1024)
+    cfg.update(over)
+    return cfg
+
+
+TALL = {"kv64": tall, "kv512": lambda: tall(dim=512, kv_lora_rank=512, rope_dim=64, qk_nope_dim=192, head_k_dim=256, v_head_dim=64)}
+
+
+def runs(rng, *spec):
+    """Tokens run by run: (count, id), or ordinary ones where the id is None."""
+    return np.concatenate([rng.integers(10, 300, n) if t is None else np.full(n, t) for n, t in spec]).astype(np.int32)
+
+
+PROMPTS = {
+    "zeros": lambda rng: runs(rng, (100, None), (200, 0), (200, None), (300, 0), (224, None)),
+    "zeros first": lambda rng: runs(rng, (200, 0), (200, None), (624, 0)),
+    "falling": lambda rng: runs(rng, (50, None), (60, 1), (90, 2), (100, 3), (52, None), (32, 1), (64, 3), (128, 2), (448, None)),
+    "small then ordinary": lambda rng: runs(rng, (352, 3), (352, 2), (300, 1), (20, None)),
+    "zeros after small": lambda rng: runs(rng, (40, None), (64, 3), (200, 0), (100, 2), (400, 0), (220, None)),
+    "scores": lambda rng: runs(rng, (1024, None)),
+}
+
+
+@pytest.mark.parametrize("name", list(TALL))
+@pytest.mark.parametrize("what", list(PROMPTS))
+def test_running_scale_matches_fp32(name, what):
+    cfg = TALL[name]()
+    g, attn = gmoe.synth_model_weights(cfg, 19)
+    g["tok_q"][0] = 0
+    for t in (1, 2, 3):
+        g["tok_s"][t] *= 2.0 ** -(16 + 20 * t)
+    if what == "scores":
+        for a in attn:
+            a["q_b_s"] *= 4.0
+    model = gmoe.Model(cfg)
+    try:
+        model.upload(g)
+        for l, a in enumerate(attn):
+            model.upload_attn(l, a)
+        toks = PROMPTS[what](np.random.default_rng(7))
+        assert toks.size == 1024
+        print(f"[case] {name}: {what}", flush=True)
+        want = run(model, toks, 0, fp32=True)
+        got = run(model, toks, 0, fp32=False)
+        assert np.isfinite(want).all()
+        assert_close(got, want, f"{name} {what}: logits", max_abs=2e-4, rel_l2=2e-5)
+        assert int(np.argmax(got)) == int(np.argmax(want)), f"{name} {what}: argmax"
+    finally:
+        model.close()
