@@ -138,20 +138,24 @@ __global__ __launch_bounds__(A16_BLOCK, 1) void k_attn_tile16(AttnTileArgs g) {
     }
     const int ntile = (r1 - r0 + A16_P - 1) / A16_P;
 
-    // a tile by DMA into stage st: A16_P rows, contiguous in the cache and in shared memory
-    // (rows past r1 are allocated: the cache's split form is padded to A16_P positions)
-    // (each wave an 18 KB run and the first wave the last KB; the DMA's offset field steps the
-    // address and the destination alike, so a base serves four)
+    // a tile by DMA into stage st: A16_P rows, contiguous in the cache and in shared memory (each
+    // wave an 18 KB run and the first wave the last KB; the DMA's offset field steps the address
+    // and the destination alike, so a base serves four). Rows past r1 hold what an earlier prompt
+    // left, and an exponential of 0 doesn't take an inf or NaN out of a sum: the buffer ends
+    // at r1, past which its loads give zeros.
     auto issue = [&](int s0, int st) {
         constexpr int KB = A16_STAGE / 1024, PER = KB / 4;
         static_assert(KB * 1024 == A16_STAGE && KB == 4 * PER + 1 && PER % 4, "whole waves of DMA, one past four equal runs");
         const uint8_t *ks = reinterpret_cast<const uint8_t *>(a.ksp + (size_t)s0 * SPL_KROW);
+        const int end = min(r1 - s0, A16_P) * SPL_KROW * 2;
         const auto *dst = (const __attribute__((address_space(3))) uint8_t *)&stg[0][0] + st * A16_STAGE;
+        auto run = [&](auto N, int kb) {
+            dma_buf<decltype(N)::value>(ks + 1024 * kb, end - 1024 * kb, 16 * lane, (const lds_void *)(dst + 1024 * kb));
+        };
 #pragma unroll
-        for (int r = 0; r + 4 <= PER; r += 4) dma_run<4>(ks + 1024 * (PER * w + r), 16 * lane, (const lds_void *)(dst + 1024 * (PER * w + r)));
-        constexpr int R = PER / 4 * 4;
-        dma_run<PER - R>(ks + 1024 * (PER * w + R), 16 * lane, (const lds_void *)(dst + 1024 * (PER * w + R)));
-        if (w == 0) dma_run<1>(ks + 1024 * (KB - 1), 16 * lane, (const lds_void *)(dst + 1024 * (KB - 1)));
+        for (int r = 0; r + 4 <= PER; r += 4) run(std::integral_constant<int, 4>{}, PER * w + r);
+        run(std::integral_constant<int, PER % 4>{}, PER * w + PER / 4 * 4);
+        if (w == 0) run(std::integral_constant<int, 1>{}, KB - 1);
     };
     issue(r0, 0);  // before the queries' loads: the two share a round trip
 

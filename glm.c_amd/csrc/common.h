@@ -67,21 +67,27 @@ __device__ static inline void dma_s(const void *base, unsigned off, const lds_vo
         asm volatile(GM_M0("%2") "global_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
 }
 // N (at most 4) consecutive pieces of 1 KB, 16 bytes per lane each: piece i from base + 1024 i
-// to dst + 1024 i, by the instruction's offset, which applies to both.
+// to dst + 1024 i, by the instruction's offset, which applies to both; zeros for what lies `end`
+// bytes or more past base (base and end uniform over the wave; a raw buffer's range check).
 template <int N>
-__device__ static inline void dma_run(const void *base, unsigned off, const lds_void *dst) {
+__device__ static inline void dma_buf(const void *base, int end, unsigned off, const lds_void *dst) {
+    typedef int i4 __attribute__((ext_vector_type(4)));
     const unsigned m0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)dst);
-#define GM_DMA "global_load_lds_dwordx4 %0, %1"
+    const uint64_t b = (uint64_t)base;
+    // base, stride 0, the buffer's bytes, 32-bit data
+    const i4 rsrc = {__builtin_amdgcn_readfirstlane((int)b), __builtin_amdgcn_readfirstlane((int)(b >> 32) & 0xffff),
+                     __builtin_amdgcn_readfirstlane(end > 0 ? end : 0), 0x00020000};
+#define GM_DMA "buffer_load_dwordx4 %0, %1, 0 offen"
     if (N == 1)
-        asm volatile(GM_M0("%2") GM_DMA ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
+        asm volatile(GM_M0("%2") GM_DMA " lds" ::"v"(off), "s"(rsrc), "s"(m0) : "memory", "m0");
     else if (N == 2)
-        asm volatile(GM_M0("%2") GM_DMA "\n\t" GM_DMA " offset:1024" ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
+        asm volatile(GM_M0("%2") GM_DMA " lds\n\t" GM_DMA " offset:1024 lds" ::"v"(off), "s"(rsrc), "s"(m0) : "memory", "m0");
     else if (N == 3)
-        asm volatile(GM_M0("%2") GM_DMA "\n\t" GM_DMA " offset:1024\n\t" GM_DMA " offset:2048" ::"v"(off), "s"(base),
+        asm volatile(GM_M0("%2") GM_DMA " lds\n\t" GM_DMA " offset:1024 lds\n\t" GM_DMA " offset:2048 lds" ::"v"(off), "s"(rsrc),
                      "s"(m0) : "memory", "m0");
     else
-        asm volatile(GM_M0("%2") GM_DMA "\n\t" GM_DMA " offset:1024\n\t" GM_DMA " offset:2048\n\t" GM_DMA
-                     " offset:3072" ::"v"(off), "s"(base), "s"(m0) : "memory", "m0");
+        asm volatile(GM_M0("%2") GM_DMA " lds\n\t" GM_DMA " offset:1024 lds\n\t" GM_DMA " offset:2048 lds\n\t" GM_DMA
+                     " offset:3072 lds" ::"v"(off), "s"(rsrc), "s"(m0) : "memory", "m0");
 #undef GM_DMA
 }
 // The block's barrier once the wave's shared-memory reads and writes are done, without

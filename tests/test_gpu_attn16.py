@@ -146,3 +146,27 @@ def test_running_scale_matches_fp32(name, what):
         assert int(np.argmax(got)) == int(np.argmax(want)), f"{name} {what}: argmax"
     finally:
         model.close()
+
+
+@pytest.mark.parametrize("name", list(TALL))
+def test_entries_past_the_batch_are_not_read(name):
+    """Token 4's embedding is NaN, and so are its cache entries and those that attend it. A
+    prompt of 100 tokens leaves them at positions 40 and up; another of 35 over the same cache
+    shares a 32-position tile with them and attends none."""
+    cfg = TALL[name]()
+    g, attn = gmoe.synth_model_weights(cfg, 19)
+    g["tok_s"][4] = np.nan
+    model = gmoe.Model(cfg)
+    try:
+        model.upload(g)
+        for l, a in enumerate(attn):
+            model.upload_attn(l, a)
+        rng = np.random.default_rng(3)
+        print(f"[case] {name}: stale NaN entries", flush=True)
+        assert np.isnan(run(model, runs(rng, (40, None), (1, 4), (59, None)), 0, fp32=False)).all()
+        toks = runs(rng, (35, None))
+        got = run(model, toks, 0, fp32=False)
+        want = run(model, toks, 0, fp32=True)
+        assert_close(got, want, f"{name}: logits", max_abs=2e-4, rel_l2=2e-5)
+    finally:
+        model.close()
