@@ -1133,18 +1133,21 @@ extern "C" int gmoe_forward(gmoe_ctx *c, int layer, int T, const float *x_in, fl
             if (rc) return rc;
         }
     } else if (grouped) {
-        // prefill: digits of xn, the per-expert lists and tiles, grouped gate/up, digits
-        // of h, grouped down, per-token combine (grouped.h)
+        // prefill: the split form of xn (here where k_rt_dots doesn't write it), the per-expert
+        // lists and tiles, grouped gate/up, the split form of h, grouped down, per-token combine
+        // (grouped.h). The native form has no profile entry of its own for a split: one record
+        // there is a product with its inputs' split, so that a layer counts one launch of each.
         const int TK = c->Tmax * K;
-        if (!split_xn) {
-            // (the native form has no entry of its own for these: counted with the product they feed)
-            pr = prof_begin(c, st, c->native ? GMOE_KERNEL_GATE_UP : GMOE_KERNEL_DIGITS);
-            hipLaunchKernelGGL(k_act_split, dim3(T), dim3(GP_BLOCK), 0, st, (const float *)c->xn, D, T, (const int *)nullptr, 0,
-                               c->xspl, c->xexp);
-            prof_end(pr, st);
-        }
         int rc = launch_dispatch(c, T, routed_on, st);
         if (rc) return rc;
+        const bool one_record = c->native;
+        pr = nullptr;
+        if (!split_xn) {
+            pr = prof_begin(c, st, one_record ? GMOE_KERNEL_GATE_UP : GMOE_KERNEL_DIGITS);
+            hipLaunchKernelGGL(k_act_split, dim3(T), dim3(GP_BLOCK), 0, st, (const float *)c->xn, D, T, (const int *)nullptr, 0,
+                               c->xspl, c->xexp);
+            if (!one_record) prof_end(pr, st);
+        }
         GroupArgs ga;
         ga.experts = L.experts;
         ga.stride = c->stride;
@@ -1168,21 +1171,21 @@ extern "C" int gmoe_forward(gmoe_ctx *c, int layer, int T, const float *x_in, fl
         ga.gs_inv = c->native ? gn_inv(c->cfg.group_size) : 0;
         const int ns = c->native ? gn_scales(c->cfg.group_size) : 0;
         const int max_tiles = (routed_on ? E + (T * K + GP_TOK - 1) / GP_TOK : 0) + (T + GP_TOK - 1) / GP_TOK;
-        pr = prof_begin(c, st, GMOE_KERNEL_GATE_UP);
+        if (split_xn || !one_record) pr = prof_begin(c, st, GMOE_KERNEL_GATE_UP);
         if (ns) launch_native_group(ns, true, dim3(F / 64, max_tiles), ga, st);
         else if (c->g16) hipLaunchKernelGGL(k_group_gu<true>, dim3(F / 64, max_tiles), dim3(GP_BLOCK), 0, st, ga);
         else hipLaunchKernelGGL(k_group_gu<false>, dim3(F / 64, max_tiles), dim3(GP_BLOCK), 0, st, ga);
         prof_end(pr, st);
         // routed rows [0, offsets[E]) and the shared rows [TK, TK + T)
-        pr = prof_begin(c, st, c->native ? GMOE_KERNEL_DOWN : GMOE_KERNEL_DIGITS);
+        pr = prof_begin(c, st, one_record ? GMOE_KERNEL_DOWN : GMOE_KERNEL_DIGITS);
         const int n1 = routed_on ? T * K : 0;
         hipLaunchKernelGGL(k_act_split, dim3(n1 + T), dim3(GP_BLOCK), 0, st, (const float *)c->hbuf, F, n1,
                            (const int *)(c->offsets + E), TK, c->hspl, c->hexp);
-        prof_end(pr, st);
+        if (!one_record) prof_end(pr, st);
         ga.aspl = c->hspl;
         ga.aexp = c->hexp;
         ga.out = c->ybuf;
-        pr = prof_begin(c, st, GMOE_KERNEL_DOWN);
+        if (!one_record) pr = prof_begin(c, st, GMOE_KERNEL_DOWN);
         if (ns) launch_native_group(ns, false, dim3(D / 64, max_tiles), ga, st);
         else if (c->g16) hipLaunchKernelGGL(k_group_down<true>, dim3(D / 64, max_tiles), dim3(GP_BLOCK), 0, st, ga);
         else hipLaunchKernelGGL(k_group_down<false>, dim3(D / 64, max_tiles), dim3(GP_BLOCK), 0, st, ga);

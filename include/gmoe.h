@@ -190,7 +190,7 @@ int gmoe_get_stats(gmoe_ctx *ctx, gmoe_stats *out);
 #define GMOE_KERNEL_DOWN 2       /* down products + combine + residual */
 #define GMOE_KERNEL_DISPATCH 3   /* per-expert token lists */
 #define GMOE_KERNEL_STACK 4      /* persistent decode kernel (T=1, all requested layers) */
-#define GMOE_KERNEL_DIGITS 5     /* prefill: activations to their int8 digit form */
+#define GMOE_KERNEL_DIGITS 5     /* prefill: activations to their split fp16 form (native form: with the product) */
 #define GMOE_KERNEL_COMBINE 6    /* prefill: per-token combine + residual */
 /* 7: unused (an earlier persistent decode kernel) */
 #define GMOE_KERNEL_RELAY 8      /* persistent decode kernel whose phases poll each other's tagged results (T=1,

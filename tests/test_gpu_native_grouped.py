@@ -52,3 +52,23 @@ def test_grouped_native(sh, T, monkeypatch):
         monkeypatch.delenv("GMOE_GROUPED_MIN_T")
         rel = np.linalg.norm(got.astype(np.float64) - one) / np.linalg.norm(one.astype(np.float64))
         assert rel <= 2e-6, f"gs={sh.gs} T={T}: {rel:.2e} from the per-token kernels"
+
+
+@pytest.mark.parametrize("E", [16, 80])
+def test_profile_counts_each_product_once(E):
+    """gmoe_profile_read of a native batch: one launch a call of gate_up and of down, with the
+    grouped kernels as with the per-token ones (T = 2), so that ms / launches is a layer's time."""
+    sh = gmoe.Shape(dim=256, moe_ffn_dim=256, n_routed_experts=E, n_experts_used=2, group_size=64)
+    ctx = gmoe.Context(sh, n_layers=2, max_tokens=64, q8_form=gmoe.GMOE_Q8_NATIVE)
+    try:
+        ctx.upload(1, gmoe.HostLayer(sh, seed=62, layer=1))
+        for T in (2, 64):  # 64 * 3 >= E + 4: grouped
+            print(f"[case] native profile E={E} T={T}", flush=True)
+            ctx.profile(True)
+            for _ in range(3):
+                gmoe.forward_host(ctx, 1, gmoe.activations(62, 2, T, sh.D))
+            ran = ctx.profile_read()
+            ctx.profile(False)
+            assert ran["gate_up"][0] == ran["down"][0] == 3, ran
+    finally:
+        ctx.close()
