@@ -1,9 +1,13 @@
 """The dense GEMMs of a prefill (k_gemm_q8) against the per-token products (k_gemv): the logits
 after a prompt prefilled in one batch and after the same prompt token by token, at column
 counts that end a 64-column chunk early (by 16, 32 and 48), at rows that end a 64-row panel
-early, at both group sizes and at token counts round the tiles' edges; and with a layer 0 wide
-enough that its gate/up product runs 64 tokens a tile (160 panels, 201 tokens). The bar is the one
-used against glm.c (max-abs 1e-2, rel-L2 1e-3, the same argmax): the two differ by rounding
+early, at both group sizes and at token counts round the tiles' edges; and at rows and tokens
+enough that each product form leaves the small products' tiles (32 tokens, two halves a block)
+for the others, on 256 CUs: gate/up at 64 tokens a tile ("wide": 160 panels, 201 tokens), the rest
+at 64 ("tall": 64 panels of attn_out, down, and q_a with kv_a, 449 tokens, 1040 or more
+columns), attn_out and q_b at 32 tokens in one half ("long": 36 panels of fewer columns), and so
+gate/up ("flat": 36 panels of 528 or 544 columns). The bar is the one used against
+glm.c (max-abs 1e-2, rel-L2 1e-3, the same argmax): the two differ by rounding
 alone, and an operand read from a wrong column by far more."""
 import numpy as np
 import pytest
@@ -17,13 +21,17 @@ pytestmark = pytest.mark.gpu
 def config(gs, ql, nope, vh, dim, hidden=0, layers=2):
     return dict(dim=dim, hidden_dim=hidden or 3 * dim, n_layers=layers, n_heads=4, vocab_size=300, q_lora_rank=ql,
                 kv_lora_rank=64, rope_dim=16, qk_nope_dim=nope, head_k_dim=nope + 16, v_head_dim=vh, group_size=gs,
-                cache_cap=256, attn_layers=layers, has_l0_ffn=1, max_batch=256)
+                cache_cap=512, attn_layers=layers, has_l0_ffn=1, max_batch=512)
 
 
 CONFIGS = {"gs16_cols48_16": config(16, 48, 16, 20, 272), "gs16_cols80_112": config(16, 112, 80, 28, 304),
            "gs32_cols32_96": config(32, 96, 32, 24, 288), "gs16_wide": config(16, 48, 16, 20, 1040, 10240, 1),
-           "gs32_wide": config(32, 96, 32, 24, 1056, 10240, 1)}
-CASES = [(name, n) for name in CONFIGS for n in ([201] if name.endswith("wide") else [8, 33])]
+           "gs32_wide": config(32, 96, 32, 24, 1056, 10240, 1),
+           "gs16_tall": config(16, 4000, 16, 260, 4096, 1040, 1), "gs32_tall": config(32, 4000, 32, 264, 4096, 1056, 1),
+           "gs16_long": config(16, 112, 560, 20, 2304, 272, 1), "gs32_long": config(32, 96, 544, 24, 2304, 288, 1),
+           "gs16_flat": config(16, 48, 16, 20, 528, 2304, 1), "gs32_flat": config(32, 96, 32, 24, 544, 2304, 1)}
+TOKENS = {"wide": [201], "tall": [449], "long": [449], "flat": [449]}
+CASES = [(name, n) for name in CONFIGS for n in TOKENS.get(name[5:], [8, 33])]
 
 
 @pytest.mark.parametrize("name,n", CASES)
