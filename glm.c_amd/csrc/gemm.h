@@ -10,9 +10,8 @@
 //                 SwiGLU pair (infer.c:1078-1080) and residual add (infer.c:1061, 1083).
 //
 // Weights stay in glm.c's row-major Q8_0 form with fp32 scales, which the decode products
-// (dense.h) read too. Per 32-column block (v_mfma_f32_16x16x32_f16, group sizes that are
-// multiples of 32) or 16-column group (v_mfma_f32_16x16x16_f16, group size 16): the
-// block's int8 weights converted to fp16 exactly, two MFMAs (hi, then lo of the inputs)
+// (dense.h) read too. Per 32-column block (v_mfma_f32_16x16x32_f16, group size 32) or
+// 16-column group (v_mfma_f32_16x16x16_f16, group size 16): the block's int8 weights converted to fp16 exactly, two MFMAs (hi, then lo of the inputs)
 // into one fp32 accumulator, and one fma applying the group's fp32 scale into the running
 // fp32 sum; 2^e at the end. The inputs carry 22 significant bits, so each product is
 // within ~2^-21 of fp32's.
@@ -20,8 +19,8 @@
 // Per-head products (k_b and v_b, whose row groups of x_rows rows read their own slice of
 // the input, x_stride apart) run as groups: a block's rows lie inside one group.
 //
-// Block order is XCD-aware: the blocks of one 64-row panel (its token tiles) are dispatched
-// on one XCD in a row, so the panel is fetched from HBM once and then read from that XCD's L2.
+// Block order is XCD-aware: the blocks of one 64-row panel (its token tiles) run on one XCD,
+// so the panel is fetched from HBM once and then read from that XCD's L2 (k_gemm_q8).
 #pragma once
 
 #include <type_traits>
@@ -423,8 +422,14 @@ __device__ __attribute__((always_inline)) static inline void qg_with_na(int na, 
 // resident together share their tokens' inputs in L2 (walking one panel's tiles before the
 // next streamed the whole input once per panel: 603 MB fetched per attn_out call of a
 // 1024-token batch, for 31.5 MB of weights and inputs).
-// What bounds it is instruction issue: a chunk's eight or sixteen MFMAs take 128 or 256 clocks of a
-// wave, and everything else in it has to stay near that. Hence scalar base addresses stepped
+// What bounds the large products is instruction issue: a chunk's eight or sixteen MFMAs take 128 or
+// 256 clocks of a wave, and everything else in it has to stay near that. Counters, shares of the
+// waves' cycles: gate/up of 1024 tokens at group size 32 (the matrix cores busy 33 % of the
+// time, 5.4 vector instructions an MFMA) 43 % issuing, 32 % ready and not issued, 25 % waiting for
+// data or a barrier; attn_out there (29 %, 5.0) 43, 28 and 29 %; gate/up of 201 tokens at group size 16
+// (35 %, 4.7) 44, 30 and 26 %. The small products wait as much as they issue, too few waves being
+// there: attn_out of 201 tokens (18 %, 5.8) 36, 23 and 40 %, k_b and v_b 18 to 37, 19 to 36 and 44 to
+// 55 %. Hence scalar base addresses stepped
 // along the rows (no vector instruction a DMA, no division by the group size), operands read
 // together, the accumulators in vector registers (launch bounds that leave the matrix cores no
 // use for their own, whose every read is an instruction). Before and after, us, with the rules
@@ -457,14 +462,23 @@ void k_gemm_q8(QgArgs a) {
 
 // Tokens per tile for n tokens and `panels` 64-row panels on n_cu compute units: 64 where that
 // leaves every CU two blocks (a chunk's weights are converted once for twice the tokens) and the
-// rows are long enough for it to tell, else 32, which is twice the blocks. 1024 tokens at group
-// size 32, 32 and 64 tokens a tile: attn_out (5120 columns) 98 and 79 us, layer 0's gate/up (2048)
-// 275 and 240, q_b (768) 34.3 and 34.0, k_b (192) 30.2 and 34.2.
+// rows are long enough for it to tell, else 32, which is twice the blocks. Both sides round the
+// lines, us, 32 and 64 tokens a tile (GLM-4.7-Flash's products):
+//   blocks, gate/up (160 panels, 2048 columns; the line at 193 tokens): group size 16, 128 tokens 52.9
+//     and 61.4, 201: 77.0 and 76.4, 256: 88.1 and 96.3 (640 blocks, 512 at once), 384: 135 and
+//     122, 1024: 332 and 294; group size 32, 128 tokens 45.0 and 45.1, 201: 69.2 and 60.1, 1024: 277 and 228;
+//   blocks, attn_out (32 panels, 5120 columns; at 961): group size 16, 896 tokens 103 and 107, 1024:
+//     108 and 108; group size 32, 768 tokens 66.2 and 66.3, 896: 84.0 and 68.1, 1024: 89.2 and 73.5;
+//   columns, 1024 tokens: k_b (192 columns) 29.8 and 38.9 at group size 16, 29.8 and 33.2 at 32; v_b
+//     (512) 33.4 and 38.8, 31.8 and 32.2; q_b (768) 41.7 and 46.9, 33.8 and 30.8.
 static inline int qg_tokens(int n, int panels, int cols, int n_cu) {
     return cols >= 1024 && (size_t)panels * ((n + 63) / 64) >= 2 * (size_t)n_cu ? 64 : 32;
 }
 // Whether the 32-token tiles' blocks run two halves of four waves, each every other chunk: where
-// there are too few blocks to give each SIMD two waves of them, which hide each other's waits. 201
-// tokens at group size 16: attn_out (224 blocks) 52 and 41 us; q_a and kv_a (147 blocks in one
-// launch) 18 us, where a launch each took 22.
+// there are too few blocks to give each SIMD two waves of them, which hide each other's waits. Us
+// with one and two halves: attn_out at group size 16, 16 tokens 37.8 and 27.3, 256: 48.6 and 37.9,
+// 448 (448 blocks) 56.6 and 57.9, 512 (512 blocks, the line) 59.4 and 60.2; at group size 32, 256
+// tokens 44.1 and 38.5, 448: 51.2 and 44.6, 512: 53.2 and 46.6; q_a and kv_a in one launch, 201 tokens 21.2
+// and 17.4 (19.4 and 15.4 at group size 32), 768 (504 blocks) 33.2 and 37.4. Short rows cross earlier:
+// v_b (512 columns), 96 tokens (240 blocks) 8.6 and 7.8, 160 (400) 10.1 and 11.2.
 static inline bool qg_halves(int n, int panels, int n_cu) { return (size_t)panels * ((n + 31) / 32) < 2 * (size_t)n_cu; }

@@ -4,11 +4,12 @@
 //
 // Per layer: the router (router.h) and the dispatch (dispatch.h, which also cuts every
 // list into tiles of GP_TOK tokens) run first. Then
-//   k_act_split    xn of every token as fp16 hi/lo with one exponent per token;
+//   k_act_split    xn of every token as fp16 hi/lo with one exponent per token (only where
+//                  k_rt_dots, which writes that form beside xn, does not run: E > 64);
 //   k_group_gu     per (tile, 64 rows of F): g and u for the tile's tokens (fp16 MFMA,
 //                  fp32 scale per 32-column block), h = silu(g) * u (infer.c:1184-1188,
 //                  1199-1202), stored per list row;
-//   k_act_split    h in the same form;
+//   k_act_split    h in the same form, the routed rows and the shared expert's in one launch;
 //   k_group_down   per (tile, 64 rows of D): y = down . h for the tile's tokens
 //                  (infer.c:1190, 1205), stored per list row;
 //   k_token_combine  x' = x + (shared + sum_k w_k y_k) per token, in glm.c's order
@@ -458,7 +459,7 @@ __global__ __launch_bounds__(GP_BLOCK, GP_OCC) void k_group_down(GroupArgs a) {
 // NS: fp32 scales a row has per chunk of GP_KC = 128 columns: 2 (group size a multiple of 64:
 // a piece's four MFMAs share one scale), 4 (of 32) or 8 (of 16: a block's halves apart).
 // Weights are read once per tile of 32 tokens where k_native_gate_up and k_native_down
-// (native.h, kept for T = 1) read them once per token and slot.
+// (native.h, which T = 1 and small batches take) read them once per token and slot.
 __host__ __device__ constexpr int gn_scales(int gs) { return gs % 64 == 0 ? 2 : gs % 32 == 0 ? 4 : 8; }
 // Group of the 16-column unit u (of a row of at most 2048 columns): u / (gs / 16) as a product.
 __host__ __device__ constexpr unsigned gn_inv(int gs) { return 65536u / (unsigned)(gs / 16) + 1; }

@@ -94,8 +94,8 @@ struct gmoe_model {
     float *x = nullptr, *q_a = nullptr, *q_full = nullptr, *kv_a = nullptr, *q_pe = nullptr, *q_abs = nullptr,
           *ctx = nullptr, *concat = nullptr, *ffh = nullptr, *logits = nullptr, *part_ctx = nullptr,
           *part_ml = nullptr, *saved = nullptr;
-    // the caches' split fp16 form for the batch attention (dense.h: ksp rows; null
-    // where the shape does not take it), cap rounded up to whole tiles of A16_P positions
+    // the caches' split fp16 form for the batch attention (dense.h: ksp rows; null where the
+    // shape does not take it), cap rounded up to whole tiles of A16_P positions
     _Float16 *ksp = nullptr;
     size_t cap32 = 0;
     // positions stale_lo .. stale_hi - 1 hold fp32 entries a decode step wrote without their
